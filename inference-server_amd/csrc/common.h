@@ -81,6 +81,11 @@ __device__ __forceinline__ v4f mfma_e4m3_exact(const v8i& a, const v8i& b) {
 // f8f6f4 MFMA (twice the bf16 rate) is kept there.
 __host__ __device__ inline bool moe_exact_accum(int H) { return H > 2048; }
 
+// Rows per tile of the LDS-tiled GEMMs of the larger batches, and rows per tile of the expert sort's
+// tile list for tile height block_m: the height that picks a GEMM, of which 128 names those.
+__host__ __device__ constexpr int moe_prefill_rows(bool exact) { return exact ? 128 : 192; }
+inline int moe_tile_rows(int block_m, bool exact) { return block_m == 128 ? moe_prefill_rows(exact) : block_m; }
+
 // silu(gate) * up on bf16 values, in the reference's rounding order: the grouped GEMM
 // output is bf16, silu(gate) is rounded to bf16, the product is rounded again
 // (TF/integrations/moe.py:509-520).  silu(g) = g / (1 + exp(-g)) with exp from v_exp_f32 (a few

@@ -558,8 +558,8 @@ int launch_down16(const GemmArgs& g2, int S, int max_tiles, bool qh, hipStream_t
 
 int moe_launch_grouped_gemms_prefill(const uint8_t* xq, const float* sx, const uint8_t* w13, const float* s13,
                                      const uint8_t* w2, const float* s2, const int32_t* perm, const int32_t* tiles,
-                                     const int32_t* n_tiles, int max_tiles, const uint16_t* topk_w, uint8_t* hq,
-                                     float* sh, uint16_t* pairs, int H, int I, int k, hipStream_t s);
+                                     const int32_t* n_tiles, int max_tiles, uint8_t* hq, float* sh, uint16_t* pairs,
+                                     int H, int I, int k, hipStream_t s);
 
 // Tile height (rows per M tile) for S pairs over E experts: 16-row tiles stream weights
 // (decode); beyond 8 pairs per expert 128-row tiles go to the LDS-tiled MFMA kernel (needs
@@ -593,8 +593,8 @@ int moe_launch_grouped_gemms(const uint8_t* xq, const float* sx, const uint8_t* 
                              int block_m, hipStream_t s, int32_t* tile_cnt, int32_t* tok_cnt, uint16_t* comb,
                              const uint16_t* residual) {
   if (block_m == 128)
-    return moe_launch_grouped_gemms_prefill(xq, sx, w13, s13, w2, s2, perm, tiles, n_tiles, max_tiles, topk_w, hq,
-                                            sh, pairs, H, I, k, s);
+    return moe_launch_grouped_gemms_prefill(xq, sx, w13, s13, w2, s2, perm, tiles, n_tiles, max_tiles, hq, sh, pairs,
+                                            H, I, k, s);
   const bool qh = block_m == 16 && down_quantises_h(S, I);
   GemmArgs g1{xq, sx, w13, s13, perm, tiles, n_tiles, nullptr, h, H, I, k, qh ? nullptr : tile_cnt, hq, sh,
               nullptr, nullptr, nullptr};

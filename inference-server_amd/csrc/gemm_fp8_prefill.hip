@@ -619,63 +619,30 @@ int device_cu_count() {
   return cus;
 }
 
-template <int MODE, bool BF = false>
+template <int MODE>
 int launch_prefill(const PrefillArgs& a, int max_tiles, hipStream_t s) {
   const long max_items = (long)max_tiles * a.n_nblk;
   long g = device_cu_count();
   if (g > max_items) g = max_items;
   g = (g + 7) / 8 * 8;
   if (g < 8) g = 8;
-  if (!BF && a.exact)
-    MOE_LAUNCH(MODE == PF_GATE_UP ? MOE_PROF_GATE_UP : MOE_PROF_DOWN, s,
-               (grouped_gemm_fp8_prefill_kernel<MODE, false, true>), dim3((unsigned)g), dim3(P_THREADS), 0, s, a);
-  else
-    MOE_LAUNCH(MODE == PF_GATE_UP ? MOE_PROF_GATE_UP : MOE_PROF_DOWN, s, (grouped_gemm_fp8_prefill_kernel<MODE, BF>),
-               dim3((unsigned)g), dim3(P_THREADS), 0, s, a);
+  MOE_LAUNCH(MODE == PF_GATE_UP ? MOE_PROF_GATE_UP : MOE_PROF_DOWN, s,
+             (grouped_gemm_fp8_prefill_kernel<MODE, false, true>), dim3((unsigned)g), dim3(P_THREADS), 0, s, a);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }
 
 }  // namespace
 
-// gate_up (with fused SiLU*up and e4m3 re-quantisation of h) then down, for block_m = 128 tiles.
-int moe_launch_grouped_gemms_prefill(const uint8_t* xq, const float* sx, const uint8_t* w13, const float* s13,
-                                     const uint8_t* w2, const float* s2, const int32_t* perm, const int32_t* tiles,
-                                     const int32_t* n_tiles, int max_tiles, const uint16_t* topk_w, uint8_t* hq,
-                                     float* sh, uint16_t* pairs, int H, int I, int k, hipStream_t s) {
-  // the DMA takes 32-bit per-lane byte offsets into the activations: rows (<= the sorted
-  // row capacity) x K must stay below 2^32
-  const long max_rows = (long)max_tiles * PBM;
-  if (max_rows * (H > I ? H : I) >= (1L << 32)) return MOE_ERR_INVALID_ARG;
-  // the cross-item DMA pipeline needs at least 4 K blocks per GEMM
-  if (H / PBK < 4 || I / PBK < 4 || H % PBN != 0) return MOE_ERR_INVALID_ARG;
-  PrefillArgs g1{xq, sx, w13, s13, perm, tiles, n_tiles, nullptr, nullptr, hq, sh, nullptr, H, I, k, I / PBK,
-                 moe_exact_accum(H)};
+// gate_up (with fused SiLU*up and e4m3 re-quantisation of h) then down on 128-row tiles, exact
+// accumulation; the caller (moe_launch_grouped_gemms_prefill) has checked the shape.
+int moe_launch_grouped_gemms_prefill_exact(const uint8_t* xq, const float* sx, const uint8_t* w13, const float* s13,
+                                           const uint8_t* w2, const float* s2, const int32_t* perm,
+                                           const int32_t* tiles, const int32_t* n_tiles, int max_tiles, uint8_t* hq,
+                                           float* sh, uint16_t* pairs, int H, int I, int k, hipStream_t s) {
+  PrefillArgs g1{xq, sx, w13, s13, perm, tiles, n_tiles, nullptr, nullptr, hq, sh, nullptr, H, I, k, I / PBK, 1};
   int rc = launch_prefill<PF_GATE_UP>(g1, max_tiles, s);
   if (rc) return rc;
-  PrefillArgs g2{hq, sh, w2, s2, perm, tiles, n_tiles, topk_w, pairs, nullptr, nullptr, nullptr, I, H, k, H / PBN,
-                 moe_exact_accum(H)};
+  PrefillArgs g2{hq, sh, w2, s2, perm, tiles, n_tiles, nullptr, pairs, nullptr, nullptr, nullptr, I, H, k, H / PBN, 1};
   return launch_prefill<PF_DOWN>(g2, max_tiles, s);
-}
-
-// Whether bf16 experts of this shape can take the 128-row tiles (bf16 K blocks are 64 deep).
-bool moe_prefill_bf16_ok(int H, int I, long max_rows) {
-  return H % PBN == 0 && H / 64 >= 4 && I / 64 >= 4 && I % MOE_GROUP == 0 &&
-         max_rows * 2 * (H > I ? H : I) < (1L << 32);
-}
-
-// The same pair of GEMMs for bf16 weights: gate_up writes bf16 h [S, I], down bf16(z) pair rows
-// (the combine applies the routing weight).
-int moe_launch_grouped_gemms_prefill_bf16(const uint16_t* x, const uint16_t* w13, const uint16_t* w2,
-                                          const int32_t* perm, const int32_t* tiles, const int32_t* n_tiles,
-                                          int max_tiles, uint16_t* h, uint16_t* pairs, int H, int I, int k,
-                                          hipStream_t s) {
-  if (!moe_prefill_bf16_ok(H, I, (long)max_tiles * PBM)) return MOE_ERR_INVALID_ARG;
-  PrefillArgs g1{(const uint8_t*)x, nullptr, (const uint8_t*)w13, nullptr, perm, tiles, n_tiles, nullptr, nullptr,
-                 nullptr, nullptr, h, H, I, k, I / PBK};
-  int rc = launch_prefill<PF_GATE_UP, true>(g1, max_tiles, s);
-  if (rc) return rc;
-  PrefillArgs g2{(const uint8_t*)h, nullptr, (const uint8_t*)w2, nullptr, perm, tiles, n_tiles, nullptr, pairs,
-                 nullptr, nullptr, nullptr, I, H, k, H / PBN};
-  return launch_prefill<PF_DOWN, true>(g2, max_tiles, s);
 }

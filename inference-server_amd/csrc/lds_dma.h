@@ -1,4 +1,4 @@
-// LDS staging helpers of the LDS-tiled grouped GEMM (gemm_fp8_prefill.hip): the swizzled 128-byte LDS row layout, MFMA fragment reads,
+// LDS staging helpers of the LDS-tiled grouped GEMMs (gemm_prefill.hip): the swizzled 128-byte LDS row layout, MFMA fragment reads,
 // global -> LDS DMA, wait / barrier and scalar table loads.
 #pragma once
 

@@ -160,6 +160,7 @@ struct ExpertsWs {
   int32_t* bucket; // 16-row tiles: expert buckets [E, T] of pair indices
   size_t total;
   int block_m;
+  int tile_rows;  // rows per tile of the tile list
   int max_tiles;
 };
 
@@ -167,6 +168,7 @@ ExpertsWs carve_experts(void* base, int T, int H, int I, int E, int k) {
   ExpertsWs w{};
   const int S = T * k;
   w.block_m = moe_gemm_block_m(S, E, H, I);
+  w.tile_rows = moe_tile_rows(w.block_m, moe_exact_accum(H));  // block_m at least, so max_tiles holds them
   w.max_tiles = moe_mi355x_align_max_tiles(S, E, w.block_m);
   WsCarver c(base);
   w.xq = c.take<uint8_t>((size_t)T * H);
@@ -211,7 +213,7 @@ int launch_experts(const void* x, const void* ids, int id_bytes, const void* wei
   if (!prepared) {
     rc = moe_launch_quant_act(x, T, H, w.xq, w.sx, s);
     if (rc) return rc;
-    rc = moe_launch_align(ids, id_bytes, S, E, w.block_m, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
+    rc = moe_launch_align(ids, id_bytes, S, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
                           w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt);
     if (rc) return rc;
   }
@@ -365,15 +367,15 @@ int block_impl(const void* x, const void* w_router, int T, int H, int I, int E, 
   const bool fused = moe_route_can_fuse_align(T, E, k);
   const bool counted = !fused && w.align_ws_bytes > 0;
   int rc = moe_launch_route(x, w_router, T, H, E, k, renorm, lg, id_out, idb, wt, b.route_ws, b.route_bytes, s,
-                            w.xq, w.sx, w.block_m, fused ? w.perm : nullptr, w.counts, w.offsets, w.tiles,
+                            w.xq, w.sx, w.tile_rows, fused ? w.perm : nullptr, w.counts, w.offsets, w.tiles,
                             w.n_tiles, counted ? (int32_t*)w.align_ws : nullptr, w.cnt, w.n_cnt);
   if (rc) return rc;
   if (counted) {
-    rc = moe_launch_align_counted(id_out, idb, T * k, E, w.block_m, (const int32_t*)w.align_ws, w.perm, w.counts,
+    rc = moe_launch_align_counted(id_out, idb, T * k, E, w.tile_rows, (const int32_t*)w.align_ws, w.perm, w.counts,
                                   w.offsets, w.tiles, w.n_tiles, s, w.cnt, w.n_cnt);
     if (rc) return rc;
   } else if (!fused) {
-    rc = moe_launch_align(id_out, idb, T * k, E, w.block_m, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
+    rc = moe_launch_align(id_out, idb, T * k, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
                           w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt);
     if (rc) return rc;
   }

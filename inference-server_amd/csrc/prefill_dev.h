@@ -1,0 +1,200 @@
+// What the LDS-tiled grouped GEMMs of the larger batches share (gemm_prefill.hip: FP8 MFMA and bf16
+// experts; gemm_prefill_exact.hip: FP8 experts accumulated exactly): arguments, work items, epilogues
+// and the launch grid.
+//
+// Tile: a few 16-row groups of one expert's sorted rows x 256 weight rows x 128-byte K blocks.
+//   gate_up: the 256 weight rows are 128 gate rows [n0, n0+128) and the matching 128 up rows
+//            [I+n0, I+n0+128), so one tile yields 128 complete h columns = one quantisation group.
+//            The epilogue computes h = silu(g)*u in the reference's bf16 rounding order and, for
+//            FP8, the per-row group amax and the e4m3 intermediate with its scale.
+//   down:    256 output columns; bf16(z) at the pair's original row t*k+j (the combine weights it).
+// Workgroup: two groups of four waves; group g owns the 16-row groups 2 m + g of the tile, wave wn of
+// a group 64 of the 256 weight rows.  Work scales with the rows a tile really holds: fragments, MFMAs
+// and epilogue of 16-row groups past its end are left out.
+#pragma once
+
+#include "common.h"
+#include "lds_dma.h"
+
+namespace {
+using namespace moe_lds;
+
+enum { PF_GATE_UP = 0, PF_DOWN = 1 };
+
+constexpr int PBN = 256;               // weight rows per tile
+constexpr int PBK = 128;               // bytes of a K block
+constexpr int P_BSLOT = PBN * PBK;     // 32 KB
+constexpr int kMaxKB = 32;             // FP8: K <= 4096
+constexpr int P_THREADS = 512;
+
+struct PrefillArgs {
+  const uint8_t* a;        // gate_up: xq [T, K] (token rows); down: hq [S, K] (sorted rows); bf16: x, h
+  const float* sa;         // activation scales [rows, K/128]
+  const uint8_t* w;        // [E, Nw, K]
+  const float* sw;         // [E, Nw/128, K/128]
+  const int32_t* perm;     // sorted row -> flat pair
+  const int32_t* tiles;    // {expert, first sorted row, rows, 0}
+  const int32_t* n_tiles;
+  uint16_t* pairs;         // down: output [S, N] by flat pair
+  uint8_t* hq;             // gate_up: e4m3 intermediate [S, N]
+  float* sh;               // gate_up: its scales [S, N/128]
+  uint16_t* h;             // bf16 weights, gate_up: the bf16 intermediate [S, N]
+  int K;                   // reduction length (elements)
+  int N;                   // gate_up: I; down: H
+  int topk;
+  int n_nblk;              // column blocks per tile: gate_up I/128, down H/256
+  int rotate;              // start each expert's K loop at another block (launch_prefill)
+};
+
+struct PfItem {
+  int e, row0, rows, nb;
+};
+
+__device__ __forceinline__ PfItem pf_item(const PrefillArgs& p, int item) {
+  const int tile = item / p.n_nblk;
+  const int4 ti = const_ld4(p.tiles, tile);
+  return {ti.x, ti.y, ti.z, item - tile * p.n_nblk};
+}
+
+// 16-row fragments of wave group g in a tile of `rows` rows, at least one (a tile of up to 16 rows
+// gives group 1 a fragment of repeated rows, whose results are never stored)
+__device__ __forceinline__ int pf_frags(int rows, int g) { return rows > 16 ? (((rows + 15) >> 4) - g + 1) >> 1 : 1; }
+
+// First K block of expert e: its K blocks are taken in the order r, r + 1, .., KB - 1, 0, .., r - 1.
+// Where the operand rows are a multiple of 4 KB long, the K block that the chip's workgroups read at
+// about the same time lies in the same few memory channels for every weight row, and experts that
+// start at different blocks spread them (weights alone, streamed in lockstep: 4.3 TB/s at 4 KB rows,
+// 5.9 at 2 KB, where nothing was gained; Qwen3-30B-A3B with bf16 experts, gate_up at 300 / 1700 tokens
+// 182 / 211 -> 144 / 190 us; Qwen3-235B-A22B, gate_up at 300 tokens 405 -> 367 us).  The order of an
+// expert's sums depends on nothing but the expert.
+__device__ __forceinline__ int pf_first_block(int e, int rotate, int KB) { return rotate ? e * 5 % KB : 0; }
+
+template <int N>
+struct Int {
+  static constexpr int value = N;
+};
+
+struct F4 {
+  float v[4];
+  __device__ __forceinline__ float& operator[](int i) { return v[i]; }
+};
+// An empty volatile asm that takes and returns v_: the value is computed before this point and the
+// volatile asm statements keep their order, which holds each MFMA and each scale FMA in its slot.
+#define PF_PIN(v_) asm volatile("" : "+v"(v_))
+
+// The epilogues.  Lane (lr, lg) of wave wn holds, for tile rows r = (2 mi + g) 16 + lr, the columns
+// 16 ni + 4 lg + q of this wave's weight rows: acc[mi][ni][q], gate fragments ni = 0, 1 with up
+// fragments 2, 3 of the same h columns wn * 32 + 16 (ni & 1) + 4 lg + q (gate_up).
+
+// gate_up, bf16 experts: h in bf16.
+template <int NM, class Acc>
+__device__ __forceinline__ void pf_store_h_bf16(Acc& acc, const PrefillArgs& p, const PfItem& it, int g, int wn, int lr,
+                                                int lg) {
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi) {
+    const int r = (2 * mi + g) * 16 + lr;
+    if (r < it.rows) {
+      uint16_t* dst = p.h + (long)(it.row0 + r) * p.N + it.nb * 128 + wn * 32 + 4 * lg;
+#pragma unroll
+      for (int ni = 0; ni < 2; ++ni) {
+        uint2 v;
+        v.x = (uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][0], acc[mi][ni + 2][0])) |
+              ((uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][1], acc[mi][ni + 2][1])) << 16);
+        v.y = (uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][2], acc[mi][ni + 2][2])) |
+              ((uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][3], acc[mi][ni + 2][3])) << 16);
+        *(uint2*)(dst + ni * 16) = v;
+      }
+    }
+  }
+}
+
+// gate_up, FP8 experts, before the group's barrier: h into acc[mi][0..1] and its row maxima over the
+// wave's 32 columns into amax (the group's [4 waves][rows], row stride `stride`).
+template <int NM, class Acc>
+__device__ __forceinline__ void pf_silu_amax(Acc& acc, float* amax, int stride, int wn, int lr, int lg) {
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi) {
+    float m = 0.f;
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float h = silu_mul_bf16(acc[mi][ni][q], acc[mi][ni + 2][q]);
+        acc[mi][ni][q] = h;
+        m = fmaxf(m, fabsf(h));
+      }
+    // the four lanes lr, lr+16, lr+32, lr+48 share the row
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    if (lg == 0) amax[wn * stride + mi * 16 + lr] = m;
+  }
+}
+
+// After it: the e4m3 codes of h and their scales.
+template <int NM, class Acc>
+__device__ __forceinline__ void pf_quant_h(Acc& acc, const float* amax, int stride, const PrefillArgs& p,
+                                           const PfItem& it, int g, int wn, int lr, int lg) {
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi) {
+    const int r = (2 * mi + g) * 16 + lr, rl = mi * 16 + lr;
+    const float am = fmaxf(fmaxf(amax[rl], amax[stride + rl]), fmaxf(amax[2 * stride + rl], amax[3 * stride + rl]));
+    const float sc = am > 0.f ? am / MOE_FP8_MAX : 1.0f;
+    if (r < it.rows) {
+      const long srow = it.row0 + r;
+      // h / s rounded as the oracle's division (div_rn): h and amax are bf16, so 448 h / amax
+      // often lands exactly on an e4m3 rounding midpoint, where h * (1 / s) (two roundings)
+      // falls on either side (0.05% of the codes differed that way)
+      uint8_t* dst = p.hq + srow * p.N + it.nb * 128 + wn * 32 + 4 * lg;
+#pragma unroll
+      for (int ni = 0; ni < 2; ++ni)
+        *(uint32_t*)(dst + ni * 16) =
+            pack4_e4m3(clamp_fp8(div_rn(acc[mi][ni][0], sc)), clamp_fp8(div_rn(acc[mi][ni][1], sc)),
+                       clamp_fp8(div_rn(acc[mi][ni][2], sc)), clamp_fp8(div_rn(acc[mi][ni][3], sc)));
+      if (wn == 0 && lg == 0) p.sh[srow * (p.N / MOE_GROUP) + it.nb] = sc;
+    }
+  }
+}
+
+// down: bf16(z) at the pairs' rows (pairs of the tile's rows in LDS).
+template <int NM, class Acc>
+__device__ __forceinline__ void pf_store_pairs(Acc& acc, const int* s_pairs, const PrefillArgs& p, const PfItem& it,
+                                               int g, int wn, int lr, int lg) {
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi) {
+    const int r = (2 * mi + g) * 16 + lr;
+    if (r < it.rows) {
+      const long pr = s_pairs[r];
+      uint16_t* dst = p.pairs + pr * p.N + it.nb * 256 + wn * 64 + 4 * lg;
+#pragma unroll
+      for (int ni = 0; ni < 4; ++ni) {
+        uint2 v;
+        v.x = (uint32_t)f32_to_bf16(acc[mi][ni][0]) | ((uint32_t)f32_to_bf16(acc[mi][ni][1]) << 16);
+        v.y = (uint32_t)f32_to_bf16(acc[mi][ni][2]) | ((uint32_t)f32_to_bf16(acc[mi][ni][3]) << 16);
+        *(uint2*)(dst + ni * 16) = v;
+      }
+    }
+  }
+}
+
+int device_cu_count() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+      cus = n;
+    else
+      cus = 256;
+  }
+  return cus;
+}
+
+// One persistent workgroup per CU, in whole rounds of the eight XCDs, at most one per work item.
+unsigned pf_grid(const PrefillArgs& a, int max_tiles) {
+  const long max_items = (long)max_tiles * a.n_nblk;
+  long grid = device_cu_count();
+  if (grid > max_items) grid = max_items;
+  grid = (grid + 7) / 8 * 8;
+  return (unsigned)(grid < 8 ? 8 : grid);
+}
+
+}  // namespace

@@ -1,0 +1,61 @@
+"""The LDS-tiled grouped GEMMs at the edges of their tiles: experts whose row counts lie around the
+16-row fragments, the two wave groups' shares and the 192- and 144-row tiles, with K loops of 4 and 5
+blocks and with rows of a multiple of 4 KB, whose K loop starts at another block for each expert."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_oracle as orc
+from tests.helpers import TOL_MAX_ABS, TOL_MEAN_REL, errors, np_f32, to_bf16, to_dev, to_f8
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 0, 15, 16, 17, 32, 33, 80, 81, 127, 129, 143, 144, 145, 160, 191, 192, 193, 289, 400]
+
+
+def pairs_of(rng, rows):
+    """One slot per token, expert e holding rows[e] of them, tokens in a random order."""
+    ids = np.repeat(np.arange(len(rows), dtype=np.int64), rows)
+    return rng.permutation(ids)[:, None]
+
+
+@pytest.mark.parametrize("kind,H,I,rows", [
+    ("fp8", 512, 512, ROWS),                      # 4 K blocks
+    ("fp8", 1024, 640, ROWS),                     # 5 K blocks in the down GEMM
+    ("fp8", 512, 4096, [145, 0, 17, 400]),        # the down GEMM's rows are 4 KB
+    ("fp8", 2304, 512, [144, 1, 145, 81, 300]),   # exact accumulation, 18 K blocks
+    ("fp8", 4096, 512, ROWS),                     # exact, gate_up's rows are 4 KB
+    ("bf16", 256, 256, ROWS),                     # 4 K blocks
+    ("bf16", 512, 384, ROWS),                     # 6 K blocks in the down GEMM
+    ("bf16", 2048, 256, ROWS),                    # gate_up's rows are 4 KB
+    ("bf16", 256, 2048, [193, 0, 17, 192, 300]),  # the down GEMM's rows are 4 KB
+])
+def test_tile_edges(pkg, dev, kind, H, I, rows):
+    rng = np.random.default_rng(H + I + len(rows))
+    E, ids = len(rows), pairs_of(rng, rows)
+    T = len(ids)
+    assert int(pkg._lib.load().moe_mi355x_block_numerics_key(T, H, I, E, 1, int(kind == "fp8"))) & 0xFFFF == 128
+    x = orc.gen_normal_bf16(rng, (T, H))
+    w = orc.round_bf16(rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32))
+    w13 = orc.gen_normal_bf16(rng, (E, 2 * I, H), 0.02)
+    w2 = orc.gen_normal_bf16(rng, (E, H, I), 0.02)
+    if kind == "fp8":
+        (q13, s13), (q2, s2) = orc.quantize_weight_fp8(w13), orc.quantize_weight_fp8(w2)
+        ref = orc.experts_fp8(x, ids, w, q13, s13, q2, s2)
+        wd = (to_f8(q13, dev), to_dev(s13, dev), to_f8(q2, dev), to_dev(s2, dev))
+        run = pkg.experts_fp8
+    else:
+        ref = orc.experts_bf16(x, ids, w, w13, w2, acc=np.float32)
+        wd = (to_bf16(w13, dev), to_bf16(w2, dev))
+        run = pkg.experts_bf16
+    out = run(to_bf16(x, dev), to_dev(ids, dev), to_bf16(w, dev), *wd)
+    max_abs, mean_rel = errors(np_f32(out), ref)
+    assert max_abs <= TOL_MAX_ABS and mean_rel <= TOL_MEAN_REL, (max_abs, mean_rel)
+    # a row's sums are taken in an order that only its expert decides: in another place of the tiles it
+    # gives the same bits
+    p = rng.permutation(T)
+    moved = run(to_bf16(x[p], dev), to_dev(ids[p], dev), to_bf16(w[p], dev), *wd)
+    assert torch.equal(moved, out[torch.from_numpy(p).to(dev)])
