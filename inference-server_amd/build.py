@@ -41,7 +41,7 @@ CFLAGS = [
 # Per-source extra flags.  The LDS-tiled prefill GEMMs keep their MFMA results in VGPRs (their
 # scale FMAs read them there) instead of AGPRs, which would need a v_accvgpr_read per element.
 EXTRA_FLAGS = {
-    "gemm_fp8_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "gemm_prefill_exact.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

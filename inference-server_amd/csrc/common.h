@@ -83,7 +83,7 @@ __host__ __device__ inline bool moe_exact_accum(int H) { return H > 2048; }
 
 // Rows per tile of the LDS-tiled GEMMs of the larger batches, and rows per tile of the expert sort's
 // tile list for tile height block_m: the height that picks a GEMM, of which 128 names those.
-__host__ __device__ constexpr int moe_prefill_rows(bool exact) { return exact ? 128 : 192; }
+__host__ __device__ constexpr int moe_prefill_rows(bool exact) { return exact ? 144 : 192; }
 inline int moe_tile_rows(int block_m, bool exact) { return block_m == 128 ? moe_prefill_rows(exact) : block_m; }
 
 // silu(gate) * up on bf16 values, in the reference's rounding order: the grouped GEMM
