@@ -15,7 +15,7 @@
 //
 // Qwen3-235B-A22B: gate_up 690 -> 523 us and down 365 -> 289 us at 2048 tokens, 462 -> 302 us (1.6 GB of
 // weights, 5.3 TB/s) and 236 -> 210 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
-// 250 us in gate_up at their full rate) and the waits of each quarter's LDS reads, below about 64 rows
+// 165 us in gate_up at their full rate) and the waits of each quarter's LDS reads, below about 64 rows
 // per expert by the stream of weights.
 //
 // Operands reach LDS by global->LDS DMA through rings of three K blocks.  One barrier per K block s,

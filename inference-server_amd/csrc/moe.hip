@@ -51,31 +51,46 @@ extern "C" size_t moe_mi355x_align_workspace_bytes(int S, int E);
 
 namespace {
 
+// How the combine gets its routing weights: none (the pair rows are weighted), eight of a token in one
+// 16-byte load (k % 8 == 0 and aligned rows), or one by one.
+enum { CW_NONE = 0, CW_VEC = 1, CW_ONE = 2 };
+
 // out[t, :] = bf16( sum_j pairs[t*k + j, :] ) with fp32 accumulation in slot order
 // (moe.py:476 view(T,k,H).sum(1)); sentinel slots (ids outside [0,E)) add zero.
-// `wts` (bf16 [T, k]) non-null: the pair rows hold bf16(z) and the routing weight is applied
-// here, bf16(bf16(z) * w), the same rounding as a weighted pair row; null: already weighted.
+// `wts` (bf16 [T, k], W != CW_NONE): the pair rows hold bf16(z) and the routing weight is applied
+// here, bf16(bf16(z) * w), the same rounding as a weighted pair row.
 // `residual` (bf16 [T, H]) non-null: out = bf16(residual + bf16(sum)), the decoder layer's
 // residual add after the MoE block (TF/models/qwen3_moe/modeling_qwen3_moe.py:347).
-__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ pairs, const void* ids,
-                                                      int id_bytes, const uint16_t* __restrict__ wts, int T,
-                                                      int k, int H, int E, const uint16_t* __restrict__ residual,
+//
+// A workgroup has up to 2048 columns of one token, so the token, its ids and its weights are uniform
+// (scalar loads) and the only vector loads are the k rows', all in flight together.  Bound by the read
+// of the pair rows: Qwen3-30B-A3B, 4096 tokens (134 MB of rows) 36.7 -> 27.5 us, 1111 tokens 14.9 -> 10.9
+// us, Qwen3-235B-A22B, 2048 tokens 38.6 -> 27.2 us, against threads that each found their token by a
+// 64-bit division and loaded its ids and weights as vectors.  Each row is read once, past the caches: the
+// 1111-token block takes 177 us, 181 with cached loads.
+template <int W>
+__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ pairs,
+                                                      const uint32_t* __restrict__ ids, int id_dwords,
+                                                      const uint16_t* __restrict__ wts, int n_cblk, int k, int H, int E,
+                                                      const uint16_t* __restrict__ residual,
                                                       uint16_t* __restrict__ out) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int per_row = H / 8;
-  if (idx >= (long)T * per_row) return;
-  const int t = (int)(idx / per_row), c8 = (int)(idx % per_row);
+  const int t = blockIdx.x / n_cblk;
+  const int c8 = (blockIdx.x - t * n_cblk) * 256 + threadIdx.x;
+  if (c8 >= H / 8) return;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   // rows are loaded unconditionally (a sentinel slot's row exists, unwritten) and masked
   // afterwards, so that the k loads are in flight together rather than one per branch
   constexpr int kUnroll = 8;
-  // eight weights of a token in one 16-byte load when the rows allow it
-  const bool wvec = wts != nullptr && (k & 7) == 0 && ((uintptr_t)wts & 15) == 0;
   for (int j0 = 0; j0 < k; j0 += kUnroll) {
     uint4 v[kUnroll];
     bool ok[kUnroll];
     float wt[kUnroll];
-    if (wvec) {
+    auto slot = [&](int u) __attribute__((always_inline)) -> long {
+      return (long)t * k + (W == CW_VEC ? j0 + u : min(j0 + u, k - 1));
+    };
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) v[u] = __builtin_bit_cast(uint4, __builtin_nontemporal_load((const v4i*)(pairs + slot(u) * H + c8 * 8)));
+    if constexpr (W == CW_VEC) {
       const uint4 w8 = *(const uint4*)(wts + (long)t * k + j0);
       const uint32_t ww[4] = {w8.x, w8.y, w8.z, w8.w};
 #pragma unroll
@@ -86,11 +101,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      const int pr = t * k + min(j0 + u, k - 1);
-      const long id = id_bytes == 8 ? (long)((const int64_t*)ids)[pr] : (long)((const int32_t*)ids)[pr];
-      ok[u] = j0 + u < k && id >= 0 && id < E;
-      if (!wvec) wt[u] = wts ? bf16_to_f32(wts[pr]) : 1.0f;
-      v[u] = *(const uint4*)(pairs + (long)pr * H + c8 * 8);
+      // 0 <= id < E: the low word, and of a 64-bit id the high word zero
+      const uint32_t lo = ids[slot(u) * id_dwords], hi = ids[slot(u) * id_dwords + id_dwords - 1];
+      ok[u] = j0 + u < k && lo < (uint32_t)E && (id_dwords == 1 || hi == 0);
+      if constexpr (W == CW_ONE) wt[u] = bf16_to_f32(wts[slot(u)]);
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
@@ -98,7 +112,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float lo = __uint_as_float(w[i] << 16), hi = __uint_as_float(w[i] & 0xffff0000u);
-        if (wts) {
+        if constexpr (W != CW_NONE) {
           lo = round_bf16(lo * wt[u]);
           hi = round_bf16(hi * wt[u]);
         }
@@ -129,10 +143,14 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
 // out = bf16(sum_j pairs[t*k + j]) in slot order (+ residual), see combine_kernel.
 int moe_launch_combine(const uint16_t* pairs, const void* ids, int id_bytes, const uint16_t* wts, int T, int k, int H,
                        int E, const uint16_t* residual, uint16_t* out, hipStream_t s) {
-  const long threads = (long)T * (H / 8);
-  MOE_RETURN_IF(!moe_grid_fits((threads + 255) / 256), MOE_ERR_INVALID_ARG);
-  MOE_LAUNCH(MOE_PROF_COMBINE, s, combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, pairs, ids,
-             id_bytes, wts, T, k, H, E, residual, out);
+  const int n_cblk = (H / 8 + 255) / 256;
+  const int threads = H / 8 < 256 ? (H / 8 + MOE_WAVE - 1) / MOE_WAVE * MOE_WAVE : 256;
+  MOE_RETURN_IF(!moe_grid_fits((long)T * n_cblk), MOE_ERR_INVALID_ARG);
+  auto kernel = wts == nullptr                                  ? combine_kernel<CW_NONE>
+                : k % 8 == 0 && ((uintptr_t)wts & 15) == 0 ? combine_kernel<CW_VEC>
+                                                                : combine_kernel<CW_ONE>;
+  MOE_LAUNCH(MOE_PROF_COMBINE, s, kernel, dim3((unsigned)((long)T * n_cblk)), dim3((unsigned)threads), 0, s, pairs,
+             (const uint32_t*)ids, id_bytes / 4, wts, n_cblk, k, H, E, residual, out);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }

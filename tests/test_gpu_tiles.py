@@ -1,4 +1,4 @@
-"""The LDS-tiled grouped GEMMs at the edges of their tiles: experts whose row counts lie around the
+"""The combine's forms, and the LDS-tiled grouped GEMMs at the edges of their tiles: experts whose row counts lie around the
 16-row fragments, the two wave groups' shares and the 192- and 144-row tiles, with K loops of 4 and 5
 blocks and with rows of a multiple of 4 KB, whose K loop starts at another block for each expert."""
 
@@ -59,3 +59,31 @@ def test_tile_edges(pkg, dev, kind, H, I, rows):
     p = rng.permutation(T)
     moved = run(to_bf16(x[p], dev), to_dev(ids[p], dev), to_bf16(w[p], dev), *wd)
     assert torch.equal(moved, out[torch.from_numpy(p).to(dev)])
+
+
+@pytest.mark.parametrize("k", [1, 8, 12, 16])
+@pytest.mark.parametrize("id_type", [torch.int32, torch.int64])
+@pytest.mark.parametrize("T,H", [(7, 256), (130, 2304)])
+def test_combine_forms(pkg, dev, T, H, k, id_type):
+    """Weights one by one (k % 8 != 0, or rows of 8 at an odd address) and eight at a time, ids of both
+    sizes with sentinels on either side of the range (for 64-bit ids also ones whose low word is an
+    expert), one and two column blocks with a remainder."""
+    rng = np.random.default_rng(T + k)
+    E, I = 16, 256
+    ids = np.argsort(rng.random((T, E)), axis=1)[:, :k].astype(np.int64)
+    ids[0, 0], ids[T // 2, -1] = -1, E
+    if id_type == torch.int64:
+        ids[1, 0], ids[2, 0] = (1 << 32) + 3, -(1 << 32) + 3
+    x = orc.gen_normal_bf16(rng, (T, H))
+    w = orc.round_bf16(rng.uniform(0.05, 0.5, (T, k)).astype(np.float32))
+    q13, s13 = orc.quantize_weight_fp8(orc.gen_normal_bf16(rng, (E, 2 * I, H), 0.02))
+    q2, s2 = orc.quantize_weight_fp8(orc.gen_normal_bf16(rng, (E, H, I), 0.02))
+    wd = (to_f8(q13, dev), to_dev(s13, dev), to_f8(q2, dev), to_dev(s2, dev))
+    ok = (ids >= 0) & (ids < E)
+    ref = orc.experts_fp8(x, np.where(ok, ids, 0), np.where(ok, w, 0.0), q13, s13, q2, s2)
+    di = torch.from_numpy(ids).to(id_type).to(dev)
+    out = pkg.experts_fp8(to_bf16(x, dev), di, to_bf16(w, dev), *wd)
+    max_abs, mean_rel = errors(np_f32(out), ref)
+    assert max_abs <= TOL_MAX_ABS and mean_rel <= TOL_MEAN_REL, (max_abs, mean_rel)
+    odd = torch.empty(T * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(T, k).copy_(to_bf16(w, dev))
+    assert torch.equal(pkg.experts_fp8(to_bf16(x, dev), di, odd, *wd), out)
