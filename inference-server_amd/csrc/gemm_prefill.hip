@@ -103,9 +103,9 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
 #pragma unroll
   for (int i = 0; i < P_NB; ++i) {
     const int br = 8 * (wave + 8 * i);
+    const int wrow = pf_weight_row(br + dma_r);
     // gate_up: tile rows 128.. are the up rows, I - 128 rows further on
-    const int wrow = MODE == PF_GATE_UP && br >= 128 ? p.N - 128 + br : br;
-    b_voff[i] = (uint32_t)((wrow + dma_r) * K + dma_lc * 16);
+    b_voff[i] = (uint32_t)((MODE == PF_GATE_UP && br >= 128 ? p.N - 128 + wrow : wrow) * K + dma_lc * 16);
   }
 
   // ---- issue side: where the next K block of the activations and of the weights is read and put ----
@@ -207,8 +207,8 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
   const v4f zero4 = {0.f, 0.f, 0.f, 0.f};
 
   // MFMA operand order: the weight fragment is the MFMA's A operand and the activation fragment its
-  // B operand, so lane l holds columns n = 4 (l >> 4) + q, q = 0..3, of token row m = l & 15.
-  // First weight row (within the tile) of fragment ni of this wave: gate_up gate rows wn*32 + 16 ni
+  // B operand, so lane l holds weight rows n = 4 (l >> 4) + q, q = 0..3, for token row m = l & 15.
+  // First LDS weight row of fragment ni of this wave: gate_up gate rows wn*32 + 16 ni
   // (ni < 2) and the matching up rows 128 + wn*32 + 16 (ni - 2); down wn*64 + 16 ni.
   struct Frags {
     v8i af[PNM], bf[4];

@@ -13,8 +13,8 @@
 // accumulators (160 registers) are what fits; what the K loop can work out anew (fresh_tid, LDS
 // addresses) is not kept in registers.
 //
-// Qwen3-235B-A22B: gate_up 690 -> 523 us and down 365 -> 289 us at 2048 tokens, 462 -> 302 us (1.6 GB of
-// weights, 5.3 TB/s) and 236 -> 210 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
+// Qwen3-235B-A22B: gate_up 690 -> 509 us and down 365 -> 279 us at 2048 tokens, 452 -> 287 us (1.6 GB of
+// weights, 5.6 TB/s) and 231 -> 168 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
 // 165 us in gate_up at their full rate) and the waits of each quarter's LDS reads, below about 64 rows
 // per expert by the stream of weights.
 //
@@ -49,7 +49,6 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = wave >> 2, wn = wave & 3;
-  const int lr = lane & 15, lg = lane >> 4;
   const int K = p.K;
   const int KB = K / PBK;
   const int Nw = MODE == PF_GATE_UP ? 2 * p.N : p.N;
@@ -81,7 +80,7 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   };
   // Quarter jj of a lane's 32 codes of a row, chunks 2 lg and 2 lg + 1 (swizzled), lies at
   // (frag_off ^ 16 (jj / 2)) + 8 (jj % 2) within a 16-row fragment group.
-  const int frag_off = lr * 128 + ((2 * lg ^ swz_key(lr)) << 4);
+  const int frag_off = (lane & 15) * 128 + ((2 * (lane >> 4) ^ swz_key(lane & 15)) << 4);
   // A wave fills weight blocks wave + 8 i: 64 rows apart, the third and fourth of gate_up among the up
   // rows, I rows after the gate rows.
   const long b_64 = 64L * K, b_128 = MODE == PF_GATE_UP ? (long)p.N * K : 128L * K;
@@ -134,7 +133,7 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   auto desc_b = [&](int j) __attribute__((always_inline)) {
     const PfItem it = pf_item(p, my_slot + j * G);
     kB = pf_first_block(it.e, p.rotate, KB);
-    pb = p.w + ((long)it.e * Nw + (long)it.nb * (MODE == PF_GATE_UP ? 128 : 256)) * K + kB * PBK;
+    pb = p.w + ((long)it.e * Nw + (long)it.nb * (MODE == PF_GATE_UP ? 128 : 256) + pf_weight_row(8 * wave)) * K + kB * PBK;
   };
 
   // DMA instruction d of a K block's activations (d == 3: their scales) and of its weights.  All of
@@ -151,17 +150,21 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
       if (ln < sa_lanes) dma_b32<0>(s_savoff[arow0 + sa_lanes * wn + ln], psa, lsa);
     }
   };
-  auto issue_b = [&](auto dc, uint32_t lb) __attribute__((always_inline)) {
+  // A lane's byte offset from its wave's weights: pf_weight_row(8 wave + dma_r) splits into the two sums.
+  auto b_voff = [&]() __attribute__((always_inline)) -> uint32_t {
+    const uint32_t l = fresh_tid(), r = (l >> 3) & 7;
+    return __umul24(pf_weight_row(r), K) + ((((l ^ r) & 7) ^ (wn & 1)) << 4);
+  };
+  auto issue_b = [&](auto dc, uint32_t v, uint32_t lb) __attribute__((always_inline)) {
     constexpr int d = decltype(dc)::value;
-    const uint32_t l = fresh_tid();
-    const uint32_t v = (l >> 3) * (uint32_t)K + ((l ^ (l >> 3) ^ ((l >> 6) & 1)) & 7) * 16;
     dma_b128<d * 8192>(v, pb + (d & 1 ? b_64 : 0) + (d & 2 ? b_128 : 0), lb);
   };
   auto issue_b_all = [&](uint32_t lb) __attribute__((always_inline)) {
-    issue_b(Int<0>{}, lb);
-    issue_b(Int<1>{}, lb);
-    issue_b(Int<2>{}, lb);
-    issue_b(Int<3>{}, lb);
+    const uint32_t v = b_voff();
+    issue_b(Int<0>{}, v, lb);
+    issue_b(Int<1>{}, v, lb);
+    issue_b(Int<2>{}, v, lb);
+    issue_b(Int<3>{}, v, lb);
   };
   constexpr int N_B = 4, N_A = 3;  // instructions of a K block; third_a waves: N_A + 1
   // To the block after the one just issued.  Past the last item its blocks are issued over again (into
@@ -195,8 +198,8 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   const v4f zero4 = {0.f, 0.f, 0.f, 0.f};
 
   // MFMA operand order: the weight fragment is the MFMA's A operand and the activation fragment its
-  // B operand, so lane l holds columns n = 4 (l >> 4) + q, q = 0..3, of token row m = l & 15.
-  // First weight row (within the tile) of fragment ni of this wave: gate_up gate rows wn*32 + 16 ni
+  // B operand, so lane l holds weight rows n = 4 (l >> 4) + q, q = 0..3, for token row m = l & 15.
+  // First LDS weight row of fragment ni of this wave: gate_up gate rows wn*32 + 16 ni
   // (ni < 2) and the matching up rows 128 + wn*32 + 16 (ni - 2); down wn*64 + 16 ni.
 
   // ---- prologue: two tables, the first K blocks ----
@@ -265,7 +268,7 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
         if constexpr (mi < NM) {
           const v8bf aw = widen(ca[mi].x, ca[mi].y);
           read_a(mi, src, off);
-          if (jj == 3) sv[mi & 1] = s_sa[sslot][arow0 + mi * 16 + lr];  // used three MFMAs on
+          if (jj == 3) sv[mi & 1] = s_sa[sslot][arow0 + mi * 16 + (lane & 15)];  // used three MFMAs on
           auto tile = [&](auto nic) __attribute__((always_inline)) {
             constexpr int ni = decltype(nic)::value, it = 4 * mi + ni;
             tx[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[ni], aw, jj == 0 ? zero4 : tx[mi][ni], 0, 0, 0);
@@ -275,10 +278,10 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
               if constexpr (it == 1 * NT / 8) issue_a(Int<1>{}, la, lsa);
               if constexpr (it == 2 * NT / 8) issue_a(Int<2>{}, la, lsa);
               if constexpr (it == 3 * NT / 8) issue_a(Int<3>{}, la, lsa);
-              if constexpr (it == 4 * NT / 8) issue_b(Int<0>{}, lb);
-              if constexpr (it == 5 * NT / 8) issue_b(Int<1>{}, lb);
-              if constexpr (it == 6 * NT / 8) issue_b(Int<2>{}, lb);
-              if constexpr (it == 7 * NT / 8) issue_b(Int<3>{}, lb);
+              if constexpr (it == 4 * NT / 8) issue_b(Int<0>{}, b_voff(), lb);
+              if constexpr (it == 5 * NT / 8) issue_b(Int<1>{}, b_voff(), lb);
+              if constexpr (it == 6 * NT / 8) issue_b(Int<2>{}, b_voff(), lb);
+              if constexpr (it == 7 * NT / 8) issue_b(Int<3>{}, b_voff(), lb);
               if constexpr (it >= 3) fold(it - 3);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -332,11 +335,19 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[mi][ni][q] = 0.f;
     int kw = pf_first_block(it.e, p.rotate, KB);  // K block of step kb
+    // whatever the previous item's epilogue had spilled of the pipeline's registers is back before the K
+    // loop, not waited for in each of its steps (behind every DMA in flight)
+    asm volatile("" : "+v"(a_voff[0]), "+v"(a_voff[1]));
+#pragma unroll
+    for (int i = 0; i < 5; ++i) asm volatile("" : "+v"(ca[i].x), "+v"(ca[i].y));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(cb[i].x), "+v"(cb[i].y));
 #pragma unroll 1
     for (int kb = 0; kb < KB; ++kb) {
       block(nmc, acc, j, kb, kw);
       if (++kw == KB) kw = 0;
     }
+    const int ln = MODE == PF_GATE_UP ? fresh_tid() & 63 : lane, lr = ln & 15, lg = ln >> 4;
     if constexpr (MODE == PF_DOWN) {
       pf_store_pairs<NM>(acc, s_perm[j % 3], p, it, g, wn, lr, lg);
     } else {

@@ -82,9 +82,18 @@ struct F4 {
 // volatile asm statements keep their order, which holds each MFMA and each scale FMA in its slot.
 #define PF_PIN(v_) asm volatile("" : "+v"(v_))
 
+// Weight row (of the tile's 256) that lies in LDS row r: within each 32, rows 8 a + 4 b + c (b < 2, c < 4)
+// lie at 16 b + 4 a + c.  A result lane holds rows 4 a + c of a 16-row fragment, c = 0..3, and with them
+// of two neighbouring fragments eight adjacent columns: half the stores, of 64 adjacent bytes a row
+// instead of 32 (Qwen3-30B-A3B, down at 4096 Zipf-routed tokens 131 -> 114 us, bf16 4096 tokens 189 -> 170,
+// bf16 1700 tokens 122 -> 117 us; gate_up's h stores are a tenth of its time and stayed level).
+__device__ __forceinline__ int pf_weight_row(int r) {
+  return (r & ~31) | ((r & 12) << 1) | ((r >> 2) & 4) | (r & 3);
+}
+
 // The epilogues.  Lane (lr, lg) of wave wn holds, for tile rows r = (2 mi + g) 16 + lr, the columns
-// 16 ni + 4 lg + q of this wave's weight rows: acc[mi][ni][q], gate fragments ni = 0, 1 with up
-// fragments 2, 3 of the same h columns wn * 32 + 16 (ni & 1) + 4 lg + q (gate_up).
+// 32 (ni / 2) + 8 lg + 4 (ni % 2) + q of this wave's 64 (down) in acc[mi][ni][q]; gate_up: of its 32 h
+// columns, the gate in fragments 0, 1 and up in 2, 3.
 
 // gate_up, bf16 experts: h in bf16.
 template <int NM, class Acc>
@@ -94,16 +103,15 @@ __device__ __forceinline__ void pf_store_h_bf16(Acc& acc, const PrefillArgs& p, 
   for (int mi = 0; mi < NM; ++mi) {
     const int r = (2 * mi + g) * 16 + lr;
     if (r < it.rows) {
-      uint16_t* dst = p.h + (long)(it.row0 + r) * p.N + it.nb * 128 + wn * 32 + 4 * lg;
+      uint16_t* dst = p.h + (long)(it.row0 + r) * p.N + it.nb * 128 + wn * 32 + 8 * lg;
+      uint32_t v[4];
 #pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        uint2 v;
-        v.x = (uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][0], acc[mi][ni + 2][0])) |
-              ((uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][1], acc[mi][ni + 2][1])) << 16);
-        v.y = (uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][2], acc[mi][ni + 2][2])) |
-              ((uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][3], acc[mi][ni + 2][3])) << 16);
-        *(uint2*)(dst + ni * 16) = v;
+      for (int q = 0; q < 4; ++q) {
+        const int ni = q >> 1, c = 2 * (q & 1);
+        v[q] = (uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][c], acc[mi][ni + 2][c])) |
+               ((uint32_t)f32_to_bf16(silu_mul_bf16(acc[mi][ni][c + 1], acc[mi][ni + 2][c + 1])) << 16);
       }
+      *(uint4*)dst = make_uint4(v[0], v[1], v[2], v[3]);
     }
   }
 }
@@ -144,12 +152,12 @@ __device__ __forceinline__ void pf_quant_h(Acc& acc, const float* amax, int stri
       // h / s rounded as the oracle's division (div_rn): h and amax are bf16, so 448 h / amax
       // often lands exactly on an e4m3 rounding midpoint, where h * (1 / s) (two roundings)
       // falls on either side (0.05% of the codes differed that way)
-      uint8_t* dst = p.hq + srow * p.N + it.nb * 128 + wn * 32 + 4 * lg;
+      uint32_t v[2];
 #pragma unroll
       for (int ni = 0; ni < 2; ++ni)
-        *(uint32_t*)(dst + ni * 16) =
-            pack4_e4m3(clamp_fp8(div_rn(acc[mi][ni][0], sc)), clamp_fp8(div_rn(acc[mi][ni][1], sc)),
-                       clamp_fp8(div_rn(acc[mi][ni][2], sc)), clamp_fp8(div_rn(acc[mi][ni][3], sc)));
+        v[ni] = pack4_e4m3(clamp_fp8(div_rn(acc[mi][ni][0], sc)), clamp_fp8(div_rn(acc[mi][ni][1], sc)),
+                           clamp_fp8(div_rn(acc[mi][ni][2], sc)), clamp_fp8(div_rn(acc[mi][ni][3], sc)));
+      *(uint2*)(p.hq + srow * p.N + it.nb * 128 + wn * 32 + 8 * lg) = make_uint2(v[0], v[1]);
       if (wn == 0 && lg == 0) p.sh[srow * (p.N / MOE_GROUP) + it.nb] = sc;
     }
   }
@@ -164,13 +172,16 @@ __device__ __forceinline__ void pf_store_pairs(Acc& acc, const int* s_pairs, con
     const int r = (2 * mi + g) * 16 + lr;
     if (r < it.rows) {
       const long pr = s_pairs[r];
-      uint16_t* dst = p.pairs + pr * p.N + it.nb * 256 + wn * 64 + 4 * lg;
+      uint16_t* dst = p.pairs + pr * p.N + it.nb * 256 + wn * 64 + 8 * lg;
 #pragma unroll
-      for (int ni = 0; ni < 4; ++ni) {
-        uint2 v;
-        v.x = (uint32_t)f32_to_bf16(acc[mi][ni][0]) | ((uint32_t)f32_to_bf16(acc[mi][ni][1]) << 16);
-        v.y = (uint32_t)f32_to_bf16(acc[mi][ni][2]) | ((uint32_t)f32_to_bf16(acc[mi][ni][3]) << 16);
-        *(uint2*)(dst + ni * 16) = v;
+      for (int s = 0; s < 2; ++s) {
+        uint32_t v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int ni = 2 * s + (q >> 1), c = 2 * (q & 1);
+          v[q] = (uint32_t)f32_to_bf16(acc[mi][ni][c]) | ((uint32_t)f32_to_bf16(acc[mi][ni][c + 1]) << 16);
+        }
+        *(uint4*)(dst + 32 * s) = make_uint4(v[0], v[1], v[2], v[3]);
       }
     }
   }
