@@ -326,28 +326,36 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
   };
 
   // ---- prologue: two tables, the first K blocks ----
-  table(0, 0);
-  if (n_my > 1) table(1, 1);
-  wait_vm<0>();
-  lds_wait_barrier();
-  desc_a(0);
-  desc_b(0);
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
+  // The weights need no table: block 0 goes out with the tables, and the K loop starts when it has
+  // landed with its activations, the next ones in flight (300 tokens of Qwen3-30B-A3B: gate_up 78.2 ->
+  // 76.1 us, down 47.1 -> 45.5 us, against waiting for the tables and then for all first blocks).
+  auto issue_a_all = [&](int b) __attribute__((always_inline)) {
     const uint32_t la = lds_a + b * (2 * P_ASLOT), lsa = lds_sa + b * (2 * PGM * 4);
     issue_a(Int<0>{}, la, lsa);
     issue_a(Int<1>{}, la, lsa);
     issue_a(Int<2>{}, la, lsa);
     issue_a(Int<3>{}, la, lsa);
     advance_a();
-    issue_b_all(lds_b + b * P_BSLOT);
-    advance_b();
-  }
+  };
+  table(0, 0);
+  if (n_my > 1) table(1, 1);
+  desc_b(0);
+  issue_b_all(lds_b);
+  advance_b();
+  wait_vm<P_NB>();  // the tables
+  lds_wait_barrier();
+  desc_a(0);
+  issue_a_all(0);
+  issue_b_all(lds_b + P_BSLOT);
+  advance_b();
+  issue_a_all(1);
   if (g == 1) {
     issue_b_all(lds_b + 2 * P_BSLOT);
     advance_b();
+    wait_vm<N_A + 2 * P_NB>();  // in flight may be block 1 and these
+  } else {
+    wait_vm<N_A + P_NB>();  // in flight may be block 1
   }
-  wait_vm<0>();
   lds_wait_barrier();
 
   int sl = 0, sb = 0;  // slots of the K block in the rings: s & 1, s % 3

@@ -203,24 +203,35 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   // (ni < 2) and the matching up rows 128 + wn*32 + 16 (ni - 2); down wn*64 + 16 ni.
 
   // ---- prologue: two tables, the first K blocks ----
-  table(0, 0);
-  if (n_my > 1) table(1, 1);
-  wait_vm<0>();
-  lds_wait_barrier();
-  desc_a(0);
-  desc_b(0);
-#pragma unroll
-  for (int b = 0; b < 3; ++b) {
+  // The weights need no table: block 0 goes out with the tables, and the K loop starts when it has
+  // landed with its activations.  K >= 4 blocks (launcher): all three of the first item.
+  auto issue_a_all = [&](int b) __attribute__((always_inline)) {
     const uint32_t la = lds_a + b * P_ASLOT, lsa = lds_sa + b * (PBM * 4);
     issue_a(Int<0>{}, la, lsa);
     issue_a(Int<1>{}, la, lsa);
     issue_a(Int<2>{}, la, lsa);
     issue_a(Int<3>{}, la, lsa);
     advance_a();
-    issue_b_all(lds_b + b * P_BSLOT);  // K >= 4 blocks (launcher): all of the first item
+  };
+  table(0, 0);
+  if (n_my > 1) table(1, 1);
+  desc_b(0);
+  issue_b_all(lds_b);
+  advance_b();
+  wait_vm<N_B>();  // the tables
+  lds_wait_barrier();
+  desc_a(0);
+  issue_a_all(0);
+#pragma unroll
+  for (int b = 1; b < 3; ++b) {
+    issue_b_all(lds_b + b * P_BSLOT);
     advance_b();
+    issue_a_all(b);
   }
-  wait_vm<0>();
+  if (third_a)  // in flight may be blocks 1 and 2
+    wait_vm<2 * (N_A + 1 + N_B)>();
+  else
+    wait_vm<2 * (N_A + N_B)>();
   lds_wait_barrier();
 
   int slot = 0, sslot = 0;  // ring slots of K block s: s % 3, and s & 3 (activation scales)
