@@ -395,4 +395,5 @@ int moe_launch_quant_act(const void* x, int R, int C, void* q, float* scales, hi
 int moe_launch_align(const void* ids, int id_bytes, int S, int E, int block_m, int32_t* perm,
                      int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                      void* workspace, size_t workspace_bytes, hipStream_t s, int32_t* zero = nullptr,
-                     int nzero = 0);
+                     int nzero = 0, const void* qx = nullptr, int qrows = 0, int qcols = 0, uint8_t* qq = nullptr,
+                     float* qs = nullptr);

@@ -229,10 +229,8 @@ int launch_experts(const void* x, const void* ids, int id_bytes, const void* wei
   const int S = T * k;
   int rc;
   if (!prepared) {
-    rc = moe_launch_quant_act(x, T, H, w.xq, w.sx, s);
-    if (rc) return rc;
     rc = moe_launch_align(ids, id_bytes, S, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
-                          w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt);
+                          w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt, x, T, H, w.xq, w.sx);
     if (rc) return rc;
   }
   // the hand-offs pay on 16-row tiles (batches up to 8 pairs per expert): fewer launches outweigh
