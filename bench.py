@@ -71,7 +71,7 @@ class Shape:
         its bf16 h round trip between the launch's workgroups is counted too).  On the 128-row
         prefill path the launch writes the e4m3 codes of h and their scales."""
         S = T * K_TOP
-        if self.prefill_path(T):  # the 128-row kernel writes the e4m3 codes of h and their scales
+        if self.prefill_path(T):  # the LDS-tiled kernel writes the e4m3 codes of h and their scales
             out = S * self.I + 4 * S * (self.I // 128)
             return n_active * self.gate_up_expert_bytes() + T * self.H + 4 * T * (self.H // 128) + out
         out = 2 * S * self.I
@@ -100,7 +100,7 @@ class Shape:
         return n_active * 2 * 3 * self.I * self.H + 2 * self.E * self.H + 4 * T * self.H
 
     def prefill_path(self, T):
-        """True where the library picks the 128-row MFMA-tiled (compute-bound) GEMMs: beyond 8
+        """True where the library picks the LDS-tiled MFMA (compute-bound) GEMMs: beyond 8
         pairs per expert, for a hidden size in 256-column tiles and both GEMMs >= 4 K blocks."""
         return T * K_TOP > 8 * self.E and self.H % 256 == 0 and self.H >= 512 and self.I >= 512
 
@@ -112,11 +112,12 @@ S235B = Shape("qwen3-235b-a22b", 4096, 1536)
 # commit a71d4f3 (FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00, KiB; the factors calibrated on a 256 MiB copy);
 # commands and per-dispatch figures in profiles/grouped_gemm_hbm_traffic.md:
 #   decode 64:            FETCH 195,261 / WRITE 768 KiB
-#   prefill 4096, Zipf:   FETCH 292,772 / WRITE 25,458 KiB
+#   prefill 4096, Zipf:   FETCH 324,585 / WRITE 25,863 KiB (build of 759266c)
 _TRAFFIC_SRC = "profiles/grouped_gemm_hbm_traffic.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, build of a71d4f3)"
+_TRAFFIC_SRC_PREFILL = _TRAFFIC_SRC.replace("a71d4f3", "759266c")
 MEASURED_GATE_UP_TRAFFIC = {
     ("qwen3-30b-a3b", 64): {"bytes": 195261 * 1024 * 2 + 768 * 1024, "source": _TRAFFIC_SRC},
-    ("qwen3-30b-a3b", 4096): {"bytes": 292772 * 1024 * 2 + 25458 * 1024, "source": _TRAFFIC_SRC},
+    ("qwen3-30b-a3b", 4096): {"bytes": 324585 * 1024 * 2 + 25863 * 1024, "source": _TRAFFIC_SRC_PREFILL},
 }
 
 
@@ -298,7 +299,7 @@ def roofline_for(shape, T, slots, n_active):
 
 def bf16_sweep_entry(pkg, torch, dev, layer, T, steps, zipf=None):
     """The bf16-expert block (the reference's default bf16 checkpoint, no FP8 requantisation):
-    decode batches are HBM-bound, the 128-row prefill tiles bf16-MFMA-bound."""
+    decode batches are HBM-bound, the LDS-tiled prefill chunks bf16-MFMA-bound."""
     shape = layer.shape
     beta = share = None
     router = layer.wr

@@ -252,15 +252,15 @@ int moe_launch_grouped_gemms_prefill_bf16(const uint16_t* x, const uint16_t* w13
 extern "C" int moe_mi355x_align_max_tiles(int S, int E, int block_m);
 
 // Tile height for the bf16 path: 16-row streaming tiles up to 8 pairs per expert; above, the
-// 128-row LDS-tiled prefill kernel where the shape allows it (30B layer, 256 tokens: 304 -> 283 us
-// against 32-row tiles, level at 129), else 32-row tiles up to 16 pairs per expert and 64 beyond.
+// LDS-tiled prefill kernel (named 128) where the shape allows it (30B layer, 256-300 tokens: 304 -> 245
+// us against 32-row tiles), else 32-row tiles up to 16 pairs per expert and 64 beyond.
 int moe_bf16_block_m(int S, int E, int H, int I) {
   if (S <= 8 * E) return 16;
   if (moe_prefill_bf16_ok(H, I, 128L * moe_mi355x_align_max_tiles(S, E, 128))) return 128;
   return S <= 16 * E ? 32 : 64;
 }
 
-// gate_up (fused SiLU*up, bf16 h) then down (weighted pair rows; on 128-row tiles bf16(z) rows
+// gate_up (fused SiLU*up, bf16 h) then down (weighted pair rows; on the LDS tiles bf16(z) rows
 // that the combine weights), bf16 weights.  With `bucket` (16-row tiles) the tile rows' pairs come
 // from the expert buckets instead of the sort's permutation.
 int moe_launch_grouped_gemms_bf16(const uint16_t* x, const uint16_t* w13, const uint16_t* w2, const int32_t* perm,

@@ -562,10 +562,11 @@ int moe_launch_grouped_gemms_prefill(const uint8_t* xq, const float* sx, const u
                                      int H, int I, int k, hipStream_t s);
 
 // Tile height (rows per M tile) for S pairs over E experts: 16-row tiles stream weights
-// (decode); beyond 8 pairs per expert 128-row tiles go to the LDS-tiled MFMA kernel (needs
-// 256-column tiles of H and at least 4 K blocks in each GEMM for its cross-item DMA pipeline):
-// from 9 to 16 pairs per expert it also beats 32-row streaming tiles (30B layer: 192 tokens
-// 158 -> 150 us, 256 tokens 161 -> 151 us, level at 129).  Shapes it cannot take stream 32-row
+// (decode); beyond 8 pairs per expert the LDS-tiled MFMA kernels take over, 128 their name here
+// (their tiles: moe_prefill_rows), which need 256-column tiles of H and at least 4 K blocks in each
+// GEMM for the cross-item DMA pipeline: from 9 to 16 pairs per expert they also beat 32-row streaming
+// tiles (30B layer: 256 tokens 161 -> 139 us), and 16-row tiles are level with them at 128 tokens
+// (137 us).  Shapes it cannot take stream 32-row
 // tiles up to 16 pairs per expert (one tile per expert for the usual loads instead of two 16-row
 // ones) and 64-row tiles above.
 int moe_gemm_block_m(int S, int E, int H, int I) {

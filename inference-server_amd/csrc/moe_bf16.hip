@@ -98,7 +98,7 @@ int bf16_experts_after_align(const void* x, const void* ids, int id_bytes, const
                                          (uint16_t*)out, bucket);
   if (rc) return rc;
   if (fused_combine) return MOE_OK;
-  // the 128-row tiles leave the routing-weight product to the combine
+  // the LDS-tiled GEMMs leave the routing-weight product to the combine
   return moe_launch_combine(w.pairs, ids, id_bytes, w.block_m == 128 ? (const uint16_t*)weights : nullptr, T, k,
                             H, E, nullptr, (uint16_t*)out, s);
 }
