@@ -8,7 +8,8 @@
 // 403 MB in 77.5 us, 5.2 TB/s), by the matrix cores and the LDS reads under them beyond.  Against one
 // 8-wave group with two register sets of fragments on 128-row tiles, experts layer at 301 tokens 145.5 ->
 // 136.9 us, uniform 2048 tokens 250 -> 216 us (its 129 .. 160-row experts were two tiles each),
-// Zipf-routed 4096 tokens 371.6 -> 370.8 us; bf16 experts, 1700 tokens 358 -> 340 us.
+// Zipf-routed 4096 tokens 371.6 -> 370.8 us; bf16 experts, 1700 tokens 359 -> 343 us (with the separate
+// combine's 6 us of it).
 //
 // The two wave groups (waves 0-3 and 4-7: one wave of each on every SIMD) run the same program half a
 // K block apart: while one issues the MFMAs of a K block (a compute phase), the other reads its next
@@ -111,10 +112,10 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
   // ---- issue side: where the next K block of the activations and of the weights is read and put ----
   uint32_t a_voff[P_NA];  // per-lane A byte offsets of the item whose activations are being issued
   uint32_t sa_voff = 0;   // per-lane activation-scale byte offset (lanes < PGM / 4)
-  const uint8_t *pa = nullptr, *pb = nullptr;
-  const float* psa = nullptr;
-  // item (of this workgroup), its K blocks not yet issued, the next of them
-  int jA = 0, leftA = KB, kA = 0, jB = 0, leftB = KB, kB = 0;
+  const uint8_t *pa = p.a, *pb = nullptr;
+  const float* psa = p.sa;
+  // item (of this workgroup) and its K blocks not yet issued
+  int jA = 0, leftA = KB, jB = 0, leftB = KB;
 
   // tables of item j into slot j % 3: pairs of its rows (rows past its end repeat the last) and the
   // weight scales of its K blocks (gate_up: gate block nb and up block I/128 + nb; down: blocks
@@ -142,15 +143,11 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
     };
 #pragma unroll
     for (int i = 0; i < P_NA; ++i) a_voff[i] = (uint32_t)(row_of(8 * (wn + 4 * i) + dma_r) * K + dma_lc * 16);
-    kA = pf_first_block(it.e, p.rotate, KB);
-    pa = p.a + kA * PBK;
-    psa = p.sa + kA;
     if constexpr (!BF) sa_voff = (uint32_t)(row_of((PGM / 4) * wn + min(lane, PGM / 4 - 1)) * KB) * 4u;
   };
   auto desc_b = [&](int j) __attribute__((always_inline)) {
     const PfItem it = pf_item(p, my_slot + j * G);
-    kB = pf_first_block(it.e, p.rotate, KB);
-    pb = p.w + ((long)it.e * Nw + (long)it.nb * (MODE == PF_GATE_UP ? 128 : 256)) * K + kB * PBK;
+    pb = p.w + ((long)it.e * Nw + (long)it.nb * (MODE == PF_GATE_UP ? 128 : 256)) * K;
   };
 
   // DMA instruction d of a K block's activations (d == P_NA: their scales) and of its weights.  All
@@ -181,24 +178,18 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
   auto advance_a = [&]() __attribute__((always_inline)) {
     pa += PBK;
     ++psa;
-    if (++kA == KB) {
-      kA = 0;
-      pa -= K;
-      psa -= KB;
-    }
     if (--leftA == 0) {
       leftA = KB;
+      pa -= K;
+      psa -= KB;
       if (jA + 1 < n_my) desc_a(++jA);
     }
   };
   auto advance_b = [&]() __attribute__((always_inline)) {
     pb += PBK;
-    if (++kB == KB) {
-      kB = 0;
-      pb -= K;
-    }
     if (--leftB == 0) {
       leftB = KB;
+      pb -= K;
       if (jB + 1 < n_my) desc_b(++jB);
     }
   };
@@ -371,13 +362,11 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
       for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[mi][ni][q] = 0.f;
-    int kw = pf_first_block(it.e, p.rotate, KB);  // K block of step kb
 #pragma unroll 1
     for (int kb = 0; kb < KB; ++kb) {
       // ---- load phase ----
       Frags f;
-      load_frags(nmc, f, sl, sb, j % 3, kw);
-      if (++kw == KB) kw = 0;
+      load_frags(nmc, f, sl, sb, j % 3, kb);
       const uint32_t lb = lds_b + (g == 0 && sb == 0 ? 2 : sb - 1 + g) * P_BSLOT;  // slot (s + 2) % 3 or (s + 3) % 3
       const uint32_t la = lds_a + sl * (2 * P_ASLOT), lsa = lds_sa + sl * (2 * PGM * 4);
       if (g == 0) {
@@ -438,7 +427,6 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_kernel(Pref
 
 template <int MODE, bool BF>
 int launch_prefill(PrefillArgs a, int max_tiles, hipStream_t s) {
-  a.rotate = (BF ? 2 : 1) * a.K % 4096 == 0;
   MOE_LAUNCH(MODE == PF_GATE_UP ? MOE_PROF_GATE_UP : MOE_PROF_DOWN, s, (grouped_gemm_prefill_kernel<MODE, BF>),
              dim3(pf_grid(a, max_tiles)), dim3(P_THREADS), 0, s, a);
   MOE_CHECK_LAUNCH();

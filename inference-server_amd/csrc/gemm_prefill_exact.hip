@@ -90,10 +90,10 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   // scales' (lanes < sa_lanes) wait in LDS, each written and read by its own wave: no registers to
   // spare, and the reload of a spilled one would wait for every DMA in flight.
   uint32_t a_voff[2];
-  const uint8_t *pa = nullptr, *pb = nullptr;
-  const float* psa = nullptr;
-  // item (of this workgroup), its K blocks not yet issued, the next of them
-  int jA = 0, leftA = KB, kA = 0, jB = 0, leftB = KB, kB = 0;
+  const uint8_t *pa = p.a, *pb = nullptr;
+  const float* psa = p.sa;
+  // item (of this workgroup) and its K blocks not yet issued
+  int jA = 0, leftA = KB, jB = 0, leftB = KB;
   // tables of item j into slot j % 3: pairs of its rows (rows past its end repeat the last) and the
   // weight scales of its K blocks (gate_up: gate block nb and up block I/128 + nb; down: blocks
   // 2 nb and 2 nb + 1, the two 128-row halves).  At most one instruction per wave.
@@ -118,22 +118,20 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
     const int* perm = s_perm[j % 3];
     const int t = fresh_tid(), ln = t & 63, dma_r = ln >> 3;
     const int dma_lc = (ln & 7) ^ ((dma_r ^ (wn & 1)) & 7);
+    int topk = p.topk;
+    asm volatile("" : "+s"(topk));  // what a division by it needs is worked out here too
     auto row_of = [&](int r) __attribute__((always_inline)) {  // operand row of this group's local row r
       const int tr = min(((2 * (r >> 4) + g) << 4) + (r & 15), it.rows - 1);
-      return MODE == PF_GATE_UP ? perm[tr] / p.topk : it.row0 + tr;
+      return MODE == PF_GATE_UP ? perm[tr] / topk : it.row0 + tr;
     };
 #pragma unroll
     for (int i = 0; i < 2; ++i) a_voff[i] = (uint32_t)(row_of(8 * (wn + 4 * i) + dma_r) * K + dma_lc * 16);
     if (third_a) s_voff2[t] = (uint32_t)(row_of(8 * (wn + 8) + dma_r) * K + dma_lc * 16);
-    kA = pf_first_block(it.e, p.rotate, KB);
-    pa = p.a + kA * PBK;
-    psa = p.sa + kA;
     if (ln < sa_lanes) s_savoff[arow0 + sa_lanes * wn + ln] = (uint32_t)(row_of(sa_lanes * wn + ln) * KB) * 4u;
   };
   auto desc_b = [&](int j) __attribute__((always_inline)) {
     const PfItem it = pf_item(p, my_slot + j * G);
-    kB = pf_first_block(it.e, p.rotate, KB);
-    pb = p.w + ((long)it.e * Nw + (long)it.nb * (MODE == PF_GATE_UP ? 128 : 256) + pf_weight_row(8 * wave)) * K + kB * PBK;
+    pb = p.w + ((long)it.e * Nw + (long)it.nb * (MODE == PF_GATE_UP ? 128 : 256) + pf_weight_row(8 * wave)) * K;
   };
 
   // DMA instruction d of a K block's activations (d == 3: their scales) and of its weights.  All of
@@ -172,24 +170,18 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
   auto advance_a = [&]() __attribute__((always_inline)) {
     pa += PBK;
     ++psa;
-    if (++kA == KB) {
-      kA = 0;
-      pa -= K;
-      psa -= KB;
-    }
     if (--leftA == 0) {
       leftA = KB;
+      pa -= K;
+      psa -= KB;
       if (jA + 1 < n_my) desc_a(++jA);
     }
   };
   auto advance_b = [&]() __attribute__((always_inline)) {
     pb += PBK;
-    if (++kB == KB) {
-      kB = 0;
-      pb -= K;
-    }
     if (--leftB == 0) {
       leftB = KB;
+      pb -= K;
       if (jB + 1 < n_my) desc_b(++jB);
     }
   };
@@ -245,7 +237,7 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
                                         : wn * 64 + ni * 16;
     cb[ni] = *(const uint2*)(s_b[sl] + brow * 128 + off);
   };
-  auto block = [&](auto nmc, auto& acc, int j, int kb, int kw) __attribute__((always_inline)) {
+  auto block = [&](auto nmc, auto& acc, int j, int kb) __attribute__((always_inline)) {
     constexpr int NM = decltype(nmc)::value, NT = 4 * NM;
     v4f tx[NM][4];
     float w0, w1, sv[2];
@@ -279,7 +271,7 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
         if constexpr (mi < NM) {
           const v8bf aw = widen(ca[mi].x, ca[mi].y);
           read_a(mi, src, off);
-          if (jj == 3) sv[mi & 1] = s_sa[sslot][arow0 + mi * 16 + (lane & 15)];  // used three MFMAs on
+          if (jj == 3) sv[mi & 1] = s_sa[sslot][arow0 + mi * 16 + (fresh_tid() & 15)];  // used three MFMAs on
           auto tile = [&](auto nic) __attribute__((always_inline)) {
             constexpr int ni = decltype(nic)::value, it = 4 * mi + ni;
             tx[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[ni], aw, jj == 0 ? zero4 : tx[mi][ni], 0, 0, 0);
@@ -318,8 +310,8 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
     };
     quarter(Int<0>{});
     quarter(Int<1>{});
-    w0 = MODE == PF_GATE_UP ? s_swt[j % 3][0][kw] : s_swt[j % 3][wn >> 1][kw];
-    w1 = MODE == PF_GATE_UP ? s_swt[j % 3][1][kw] : 0.f;
+    w0 = MODE == PF_GATE_UP ? s_swt[j % 3][0][kb] : s_swt[j % 3][wn >> 1][kb];
+    w1 = MODE == PF_GATE_UP ? s_swt[j % 3][1][kb] : 0.f;
     quarter(Int<2>{});
     if (third_a)
       wait_vm<N_A + 1 + N_B>();
@@ -345,7 +337,6 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
       for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[mi][ni][q] = 0.f;
-    int kw = pf_first_block(it.e, p.rotate, KB);  // K block of step kb
     // whatever the previous item's epilogue had spilled of the pipeline's registers is back before the K
     // loop, not waited for in each of its steps (behind every DMA in flight)
     asm volatile("" : "+v"(a_voff[0]), "+v"(a_voff[1]));
@@ -354,11 +345,8 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
 #pragma unroll
     for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(cb[i].x), "+v"(cb[i].y));
 #pragma unroll 1
-    for (int kb = 0; kb < KB; ++kb) {
-      block(nmc, acc, j, kb, kw);
-      if (++kw == KB) kw = 0;
-    }
-    const int ln = MODE == PF_GATE_UP ? fresh_tid() & 63 : lane, lr = ln & 15, lg = ln >> 4;
+    for (int kb = 0; kb < KB; ++kb) block(nmc, acc, j, kb);
+    const int ln = fresh_tid() & 63, lr = ln & 15, lg = ln >> 4;
     if constexpr (MODE == PF_DOWN) {
       pf_store_pairs<NM>(acc, s_perm[j % 3], p, it, g, wn, lr, lg);
     } else {
@@ -391,7 +379,6 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
 
 template <int MODE>
 int launch_prefill_exact(PrefillArgs a, int max_tiles, hipStream_t s) {
-  a.rotate = a.K % 4096 == 0;
   MOE_LAUNCH(MODE == PF_GATE_UP ? MOE_PROF_GATE_UP : MOE_PROF_DOWN, s, grouped_gemm_prefill_exact_kernel<MODE>,
              dim3(pf_grid(a, max_tiles)), dim3(P_THREADS), 0, s, a);
   MOE_CHECK_LAUNCH();

@@ -43,7 +43,6 @@ struct PrefillArgs {
   int N;                   // gate_up: I; down: H
   int topk;
   int n_nblk;              // column blocks per tile: gate_up I/128, down H/256
-  int rotate;              // start each expert's K loop at another block (launch_prefill)
 };
 
 struct PfItem {
@@ -59,15 +58,6 @@ __device__ __forceinline__ PfItem pf_item(const PrefillArgs& p, int item) {
 // 16-row fragments of wave group g in a tile of `rows` rows, at least one (a tile of up to 16 rows
 // gives group 1 a fragment of repeated rows, whose results are never stored)
 __device__ __forceinline__ int pf_frags(int rows, int g) { return rows > 16 ? (((rows + 15) >> 4) - g + 1) >> 1 : 1; }
-
-// First K block of expert e: its K blocks are taken in the order r, r + 1, .., KB - 1, 0, .., r - 1.
-// Where the operand rows are a multiple of 4 KB long, the K block that the chip's workgroups read at
-// about the same time lies in the same few memory channels for every weight row, and experts that
-// start at different blocks spread them (weights alone, streamed in lockstep: 4.3 TB/s at 4 KB rows,
-// 5.9 at 2 KB, where nothing was gained; Qwen3-30B-A3B with bf16 experts, gate_up at 300 / 1700 tokens
-// 182 / 211 -> 144 / 190 us; Qwen3-235B-A22B, gate_up at 300 tokens 405 -> 367 us).  The order of an
-// expert's sums depends on nothing but the expert.
-__device__ __forceinline__ int pf_first_block(int e, int rotate, int KB) { return rotate ? e * 5 % KB : 0; }
 
 template <int N>
 struct Int {

@@ -1,6 +1,6 @@
 """The combine's forms, and the LDS-tiled grouped GEMMs at the edges of their tiles: experts whose row counts lie around the
 16-row fragments, the two wave groups' shares and the 192- and 144-row tiles, with K loops of 4 and 5
-blocks and with rows of a multiple of 4 KB, whose K loop starts at another block for each expert."""
+blocks and with rows of a multiple of 4 KB."""
 
 from __future__ import annotations
 
@@ -87,3 +87,43 @@ def test_combine_forms(pkg, dev, T, H, k, id_type):
     assert max_abs <= TOL_MAX_ABS and mean_rel <= TOL_MEAN_REL, (max_abs, mean_rel)
     odd = torch.empty(T * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(T, k).copy_(to_bf16(w, dev))
     assert torch.equal(pkg.experts_fp8(to_bf16(x, dev), di, odd, *wd), out)
+
+
+@pytest.mark.parametrize("kind,H,I", [
+    ("fp8", 512, 512),
+    ("fp8", 512, 4096),   # the down GEMM's rows are 4 KB
+    ("bf16", 2048, 256),  # gate_up's rows are 4 KB
+    ("bf16", 256, 2048),  # the down GEMM's rows are 4 KB
+])
+def test_expert_index_leaves_the_bits(pkg, dev, kind, H, I):
+    """A pair's bits depend on its expert's weights, not on the expert's index in the call: the same
+    experts in another order, and a share of them under local indices (sentinels for the others)."""
+    rows = [40, 1, 150, 17, 200, 33]
+    rng = np.random.default_rng(H + I)
+    E, ids = len(rows), pairs_of(rng, rows)
+    T = len(ids)
+    x = to_bf16(orc.gen_normal_bf16(rng, (T, H)), dev)
+    w = to_bf16(orc.round_bf16(rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32)), dev)
+    w13 = orc.gen_normal_bf16(rng, (E, 2 * I, H), 0.02)
+    w2 = orc.gen_normal_bf16(rng, (E, H, I), 0.02)
+    if kind == "fp8":
+        (q13, s13), (q2, s2) = orc.quantize_weight_fp8(w13), orc.quantize_weight_fp8(w2)
+        wd = (to_f8(q13, dev), to_dev(s13, dev), to_f8(q2, dev), to_dev(s2, dev))
+        run = pkg.experts_fp8
+    else:
+        wd = (to_bf16(w13, dev), to_bf16(w2, dev))
+        run = pkg.experts_bf16
+
+    def take(order):
+        """The call with the experts of ``order`` alone, in that order."""
+        local = np.full(E, -1, dtype=np.int64)
+        local[order] = np.arange(len(order))
+        sel = torch.as_tensor(order, device=dev)
+        part = [t.view(torch.uint8)[sel].view(t.dtype) if t.dtype == torch.float8_e4m3fn else t[sel] for t in wd]
+        return run(x, to_dev(local[ids], dev), w, *part)
+
+    whole = take(list(range(E)))
+    assert torch.equal(take([3, 0, 5, 1, 2, 4]), whole)
+    share = take([2, 4, 5])
+    mine = to_dev(np.isin(ids[:, 0], [2, 4, 5]), dev)
+    assert torch.equal(share[mine], whole[mine]) and not share[~mine].any()
