@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "moe_mi355x.h"
+#include "prefill_rows.h"
 
 #define MOE_WAVE 64
 #define MOE_GROUP 128      // quantisation group / block size
@@ -81,9 +82,8 @@ __device__ __forceinline__ v4f mfma_e4m3_exact(const v8i& a, const v8i& b) {
 // f8f6f4 MFMA (twice the bf16 rate) is kept there.
 __host__ __device__ inline bool moe_exact_accum(int H) { return H > 2048; }
 
-// Rows per tile of the LDS-tiled GEMMs of the larger batches, and rows per tile of the expert sort's
-// tile list for tile height block_m: the height that picks a GEMM, of which 128 names those.
-__host__ __device__ constexpr int moe_prefill_rows(bool exact) { return exact ? 144 : 192; }
+// Rows per tile of the expert sort's tile list for tile height block_m: the height that picks a GEMM, of
+// which 128 names the LDS-tiled ones of the larger batches.
 inline int moe_tile_rows(int block_m, bool exact) { return block_m == 128 ? moe_prefill_rows(exact) : block_m; }
 
 // silu(gate) * up on bf16 values, in the reference's rounding order: the grouped GEMM

@@ -13,8 +13,8 @@
 // accumulators (160 registers) are what fits; what the K loop can work out anew (fresh_tid, LDS
 // addresses) is not kept in registers.
 //
-// Qwen3-235B-A22B: gate_up 690 -> 509 us and down 365 -> 279 us at 2048 tokens, 452 -> 287 us (1.6 GB of
-// weights, 5.6 TB/s) and 231 -> 168 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
+// Qwen3-235B-A22B: gate_up 706 -> 545 us and down 376 -> 277 us at 2048 tokens, 480 -> 334 us (1.6 GB of
+// weights, 4.8 TB/s) and 245 -> 156 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
 // 165 us in gate_up at their full rate) and the waits of each quarter's LDS reads, below about 64 rows
 // per expert by the stream of weights.
 //
@@ -32,9 +32,10 @@
 namespace {
 
 constexpr int PBM = moe_prefill_rows(true);  // rows per tile: nine 16-row groups, five of wave group 0
-constexpr int PGM = 80;                // rows of wave group 0 (group 1: 64)
+constexpr int PGM = pf_group_row0(PBM, 1);  // rows of wave group 0 (group 1: 64)
 constexpr int P_ASLOT = PBM * PBK;     // 18 KB: group 0's rows, then group 1's
-static_assert(PBM == 144, "9 row groups");
+constexpr int P_FRAGS1 = pf_group_frags(PBM, 1);  // fragments of a wave of group 1; group 0 has one more
+static_assert(PGM == 80 && P_FRAGS1 == 4, "9 row groups");
 
 template <int MODE>
 __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kernel(PrefillArgs p) {
@@ -228,9 +229,10 @@ __global__ __launch_bounds__(P_THREADS, 1) void grouped_gemm_prefill_exact_kerne
 
   int slot = 0, sslot = 0;  // ring slots of K block s: s % 3, and s & 3 (activation scales)
 
-  uint2 ca[5], cb[4];  // codes of one quarter of the fragments
+  uint2 ca[5] = {}, cb[4];  // codes of one quarter of the fragments
   auto read_a = [&](int mi, int sl, int off) __attribute__((always_inline)) {
-    ca[mi] = *(const uint2*)(s_a[sl] + arow0 * PBK + mi * 16 * 128 + off);
+    if (mi < P_FRAGS1 || g == 0)  // group 1's part of the slot ends after four
+      ca[mi] = *(const uint2*)(s_a[sl] + arow0 * PBK + mi * 16 * 128 + off);
   };
   auto read_b = [&](int ni, int sl, int off) __attribute__((always_inline)) {
     const int brow = MODE == PF_GATE_UP ? (ni < 2 ? wn * 32 + ni * 16 : 128 + wn * 32 + (ni - 2) * 16)

@@ -92,6 +92,7 @@ def test_combine_forms(pkg, dev, T, H, k, id_type):
 @pytest.mark.parametrize("kind,H,I", [
     ("fp8", 512, 512),
     ("fp8", 512, 4096),   # the down GEMM's rows are 4 KB
+    ("fp8", 4096, 512),   # exact accumulation
     ("bf16", 2048, 256),  # gate_up's rows are 4 KB
     ("bf16", 256, 2048),  # the down GEMM's rows are 4 KB
 ])
