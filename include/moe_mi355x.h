@@ -179,6 +179,13 @@ int moe_mi355x_block_fp8_noalloc(const void* x, const void* w_router, int T, int
 long long moe_mi355x_block_numerics_key(int T, int H, int I, int E, int k, int fp8);
 
 /*
+ * Rows per tile of one expert's sorted rows in the expert GEMMs of the FP8 (fp8 != 0) or the bf16
+ * entry points, for a routing that cuts into tiles_128 tiles of at most 128 rows (each expert's rows on
+ * their own).  No result depends on it.  0 for unsupported shapes.  A query (host only).
+ */
+int moe_mi355x_experts_tile_rows(int T, int H, int I, int E, int k, int fp8, int tiles_128);
+
+/*
  * Paged GQA decode attention, one new token per sequence (the attention of a decode step of
  * Qwen3MoeAttention.forward, TF/models/qwen3_moe/modeling_qwen3_moe.py:151-191, with
  * eager_attention_forward :96-119): for query head h of sequence b, over the keys

@@ -1,5 +1,5 @@
 // Expert sort / align: stable counting sort of the T*k (token, slot) pairs by
-// expert id, per-expert counts and offsets, and the block_m-row tile list the
+// expert id, per-expert counts and offsets, and the list of row tiles the
 // grouped GEMMs iterate over.
 //
 // Reference: TF/integrations/moe.py:389-403 (torch.sort, histc, cumsum).
@@ -37,7 +37,7 @@ __device__ __forceinline__ void quant_part(const QuantPart& qp, int block) {
 
 // Whole align in one workgroup (small S: decode batches).
 __global__ __launch_bounds__(kChunk) void align_single_kernel(const void* ids, int id_bytes, int S, int E,
-                                                              int block_m, int32_t* perm, int32_t* counts,
+                                                              TileRows tile_rows, int32_t* perm, int32_t* counts,
                                                               int32_t* offsets, int32_t* tiles,
                                                               int32_t* n_tiles, int32_t* zero, int nzero,
                                                               QuantPart qp) {
@@ -49,14 +49,15 @@ __global__ __launch_bounds__(kChunk) void align_single_kernel(const void* ids, i
   __shared__ int s_cnt[kBuckets];
   __shared__ int s_off[kBuckets];
   __shared__ int s_toff[kBuckets];
+  __shared__ int s_rows;
   __shared__ int s_wcnt[kWaves][kBuckets];
   for (int e = threadIdx.x; e <= E; e += blockDim.x) s_cnt[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < S; i += blockDim.x) atomicAdd(&s_cnt[bucket_of(ids, id_bytes, i, E)], 1);
   __syncthreads();
-  scan_counts(s_cnt, E, block_m, s_off, s_toff);
+  scan_counts(s_cnt, E, tile_rows, s_off, s_toff, &s_rows);
   __syncthreads();
-  emit_meta(s_cnt, s_off, s_toff, E, block_m, counts, offsets, tiles, n_tiles);
+  emit_meta(s_cnt, s_off, s_toff, E, s_rows, counts, offsets, tiles, n_tiles);
   // s_off doubles as the running base from here on; s_off[E] starts the sentinel tail
   for (int c0 = 0; c0 < S; c0 += kChunk) scatter_chunk(ids, id_bytes, S, E, c0, s_off, s_wcnt, perm);
 }
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(kChunk) void align_count_kernel(const void* ids, in
 // chunk's starting slot per expert = offset of the expert + counts of the earlier chunks),
 // workgroup 0 writes counts, offsets and the tile list, and each places its chunk stably.
 __global__ __launch_bounds__(kChunk) void align_scan_scatter_kernel(const void* ids, int id_bytes, int S, int E,
-                                                                    int block_m, const int32_t* __restrict__ bc,
+                                                                    TileRows tile_rows, const int32_t* __restrict__ bc,
                                                                     int nb, int32_t* perm, int32_t* counts,
                                                                     int32_t* offsets, int32_t* tiles,
                                                                     int32_t* n_tiles, int32_t* zero, int nzero) {
@@ -89,6 +90,7 @@ __global__ __launch_bounds__(kChunk) void align_scan_scatter_kernel(const void* 
   __shared__ int s_cnt[kBuckets];
   __shared__ int s_off[kBuckets];
   __shared__ int s_toff[kBuckets];
+  __shared__ int s_rows;
   __shared__ int s_base[kBuckets];
   __shared__ int s_wcnt[kWaves][kBuckets];
   const int b = blockIdx.x;
@@ -104,9 +106,9 @@ __global__ __launch_bounds__(kChunk) void align_scan_scatter_kernel(const void* 
     s_base[e] = pre;
   }
   __syncthreads();
-  scan_counts(s_cnt, E, block_m, s_off, s_toff);
+  scan_counts(s_cnt, E, tile_rows, s_off, s_toff, &s_rows);
   __syncthreads();
-  if (b == 0) emit_meta(s_cnt, s_off, s_toff, E, block_m, counts, offsets, tiles, n_tiles);
+  if (b == 0) emit_meta(s_cnt, s_off, s_toff, E, s_rows, counts, offsets, tiles, n_tiles);
   for (int e = threadIdx.x; e <= E; e += blockDim.x) s_base[e] += s_off[e];
   __syncthreads();
   scatter_chunk(ids, id_bytes, S, E, b * kChunk, s_base, s_wcnt, perm);
@@ -125,7 +127,7 @@ extern "C" size_t moe_mi355x_align_workspace_bytes(int S, int E) {
   return moe_align_up(nb * (E + 1) * sizeof(int32_t), 256);
 }
 
-int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, int block_m, const int32_t* bc,
+int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, TileRows tile_rows, const int32_t* bc,
                              int32_t* perm, int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                              hipStream_t s, int32_t* zero, int nzero);
 
@@ -133,7 +135,7 @@ int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, int bl
 //
 // `qx` non-null: the activations qx bf16 [qrows, qcols] are quantised in the first launch too (qq, qs as
 // moe_launch_quant_act's).
-int moe_launch_align(const void* ids, int id_bytes, int S, int E, int block_m, int32_t* perm,
+int moe_launch_align(const void* ids, int id_bytes, int S, int E, TileRows tile_rows, int32_t* perm,
                      int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles, void* workspace,
                      size_t workspace_bytes, hipStream_t s, int32_t* zero, int nzero, const void* qx, int qrows,
                      int qcols, uint8_t* qq, float* qs) {
@@ -142,7 +144,7 @@ int moe_launch_align(const void* ids, int id_bytes, int S, int E, int block_m, i
   MOE_RETURN_IF(!moe_grid_fits(qblocks + (S + kChunk - 1) / kChunk), MOE_ERR_INVALID_ARG);
   if (S <= kAlignOneWgMaxS) {
     MOE_LAUNCH(MOE_PROF_ALIGN, s, align_single_kernel, dim3((unsigned)(1 + qblocks)), dim3(kChunk), 0, s, ids,
-               id_bytes, S, E, block_m, perm, counts, offsets, tiles, n_tiles, zero, nzero, qp);
+               id_bytes, S, E, tile_rows, perm, counts, offsets, tiles, n_tiles, zero, nzero, qp);
     MOE_CHECK_LAUNCH();
     return MOE_OK;
   }
@@ -152,18 +154,18 @@ int moe_launch_align(const void* ids, int id_bytes, int S, int E, int block_m, i
   MOE_LAUNCH(MOE_PROF_ALIGN, s, align_count_kernel, dim3((unsigned)(nb + qblocks)), dim3(kChunk), 0, s, ids, id_bytes, S,
              E, bc, nb, qp);
   MOE_CHECK_LAUNCH();
-  return moe_launch_align_counted(ids, id_bytes, S, E, block_m, bc, perm, counts, offsets, tiles, n_tiles, s, zero,
+  return moe_launch_align_counted(ids, id_bytes, S, E, tile_rows, bc, perm, counts, offsets, tiles, n_tiles, s, zero,
                                   nzero);
 }
 
 // The rest of the large-S align once the chunk histograms bc [nb, E + 1] are filled (by
 // align_count_kernel, or by the top-k kernel of the block path).
-int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, int block_m, const int32_t* bc,
+int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, TileRows tile_rows, const int32_t* bc,
                              int32_t* perm, int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                              hipStream_t s, int32_t* zero, int nzero) {
   const int nb = (S + kChunk - 1) / kChunk;
   MOE_LAUNCH(MOE_PROF_ALIGN, s, align_scan_scatter_kernel, dim3(nb), dim3(kChunk), 0, s, ids, id_bytes, S, E,
-             block_m, bc, nb, perm, counts, offsets, tiles, n_tiles, zero, nzero);
+             tile_rows, bc, nb, perm, counts, offsets, tiles, n_tiles, zero, nzero);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }
@@ -178,6 +180,6 @@ extern "C" int moe_mi355x_align(const void* ids, int id_bytes, int T, int k, int
   MOE_RETURN_IF(S > (1L << 30), MOE_ERR_INVALID_ARG);
   MOE_RETURN_IF(S > 0 && (!ids || !perm || !tiles), MOE_ERR_INVALID_ARG);
   MOE_RETURN_IF(!moe_aligned16(tiles), MOE_ERR_ALIGNMENT);
-  return moe_launch_align(ids, id_bytes, (int)S, E, block_m, perm, counts, offsets, tiles, n_tiles, workspace,
+  return moe_launch_align(ids, id_bytes, (int)S, E, {block_m, block_m, 0}, perm, counts, offsets, tiles, n_tiles, workspace,
                           workspace_bytes, (hipStream_t)stream);
 }

@@ -21,8 +21,9 @@ constexpr int kSingleMaxS = 4096;  // pairs the one-workgroup top-k + sort kerne
 // slots 13.5 -> 7.6 us.
 constexpr int kAlignOneWgMaxS = 2048;
 
-// Exclusive scans of counts and of ceil(count / block_m) over experts; wave 0 of the block.
-__device__ void scan_counts(const int* s_cnt, int E, int block_m, int* s_off, int* s_toff) {
+// Picks the rows per tile (s_rows[0]), then exclusive scans of counts and of ceil(count / rows) over
+// experts; wave 0 of the block.
+__device__ void scan_counts(const int* s_cnt, int E, TileRows tr, int* s_off, int* s_toff, int* s_rows) {
   const int lane = threadIdx.x & 63;
   if ((threadIdx.x >> 6) != 0) return;
   int c[4], t[4], sc = 0, st = 0;
@@ -30,7 +31,19 @@ __device__ void scan_counts(const int* s_cnt, int E, int block_m, int* s_off, in
   for (int q = 0; q < 4; ++q) {
     const int e = lane * 4 + q;
     c[q] = e < E ? s_cnt[e] : 0;
-    t[q] = (c[q] + block_m - 1) / block_m;
+  }
+  int rows = tr.rows;
+  if (tr.low_tiles > 0) {  // kernel-uniform
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) n += (c[q] + tr.low - 1) / tr.low;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d, MOE_WAVE);
+    rows = moe_pick_rows(tr, n);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    t[q] = (c[q] + rows - 1) / rows;
     sc += c[q];
     st += t[q];
   }
@@ -57,6 +70,7 @@ __device__ void scan_counts(const int* s_cnt, int E, int block_m, int* s_off, in
   if (lane == 63) {
     s_off[E] = ic;
     s_toff[E] = it;
+    s_rows[0] = rows;
   }
 }
 
@@ -67,7 +81,7 @@ __device__ __forceinline__ void zero_counters(int32_t* zero, int n) {
 }
 
 // Writes counts, offsets and the tile list from the scanned LDS arrays.
-__device__ void emit_meta(const int* s_cnt, const int* s_off, const int* s_toff, int E, int block_m,
+__device__ void emit_meta(const int* s_cnt, const int* s_off, const int* s_toff, int E, int rows,
                           int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles) {
   for (int e = threadIdx.x; e <= E; e += blockDim.x) {
     offsets[e] = s_off[e];
@@ -78,8 +92,8 @@ __device__ void emit_meta(const int* s_cnt, const int* s_off, const int* s_toff,
     const int c = s_cnt[e];
     counts[e] = c;
     int tix = s_toff[e];
-    for (int r = 0; r < c; r += block_m, ++tix) {
-      int4 v = make_int4(e, s_off[e] + r, min(block_m, c - r), 0);
+    for (int r = 0; r < c; r += rows, ++tix) {
+      int4 v = make_int4(e, s_off[e] + r, min(rows, c - r), 0);
       *(int4*)(tiles + 4 * tix) = v;
     }
   }

@@ -82,9 +82,34 @@ __device__ __forceinline__ v4f mfma_e4m3_exact(const v8i& a, const v8i& b) {
 // f8f6f4 MFMA (twice the bf16 rate) is kept there.
 __host__ __device__ inline bool moe_exact_accum(int H) { return H > 2048; }
 
-// Rows per tile of the expert sort's tile list for tile height block_m: the height that picks a GEMM, of
-// which 128 names the LDS-tiled ones of the larger batches.
-inline int moe_tile_rows(int block_m, bool exact) { return block_m == 128 ? moe_prefill_rows(exact) : block_m; }
+// Rows per tile of the expert sort's tile list: `rows`, or `low` where those give at most low_tiles tiles.
+struct TileRows {
+  int rows, low, low_tiles;
+};
+
+// CUs of the current device (the first call's: all GPUs of a node are alike).
+inline int moe_cu_count() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    return hipGetDevice(&dev) == hipSuccess &&
+                   hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0
+               ? n
+               : 256;
+  }();
+  return cus;
+}
+
+// ... for tile height block_m: the height that picks a GEMM, of which 128 names the LDS-tiled ones of the
+// larger batches.  No tile is lower than block_m (unless its expert ends), so block_m bounds their number.
+inline TileRows moe_tile_rows(int block_m, bool exact, int H, int I) {
+  if (block_m != 128) return {block_m, block_m, 0};
+  return {moe_prefill_rows(exact), kPrefillLowRows, moe_prefill_low_tiles(exact, H, I, moe_cu_count())};
+}
+
+// The rows of a list that has n_low tiles of tr.low rows.
+__host__ __device__ inline int moe_pick_rows(const TileRows& tr, int n_low) {
+  return n_low <= tr.low_tiles ? tr.low : tr.rows;
+}
 
 // silu(gate) * up on bf16 values, in the reference's rounding order: the grouped GEMM
 // output is bf16, silu(gate) is rounded to bf16, the product is rounded again
@@ -392,7 +417,7 @@ void moe_prof_end(int id, hipStream_t s);
 // Internal launchers shared between translation units.
 int moe_launch_quant_act(const void* x, int R, int C, void* q, float* scales, hipStream_t s,
                          int slot = MOE_PROF_QUANT_ACT);
-int moe_launch_align(const void* ids, int id_bytes, int S, int E, int block_m, int32_t* perm,
+int moe_launch_align(const void* ids, int id_bytes, int S, int E, TileRows tile_rows, int32_t* perm,
                      int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                      void* workspace, size_t workspace_bytes, hipStream_t s, int32_t* zero = nullptr,
                      int nzero = 0, const void* qx = nullptr, int qrows = 0, int qcols = 0, uint8_t* qq = nullptr,

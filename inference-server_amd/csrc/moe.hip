@@ -38,10 +38,10 @@ int moe_launch_grouped_gemms_buckets(const uint8_t* xq, const float* sx, const u
                                      const uint16_t* residual);
 int moe_launch_route(const void* x, const void* w_router, int T, int H, int E, int k, int renorm,
                      void* logits, void* ids, int id_bytes, void* weights, void* workspace,
-                     size_t workspace_bytes, hipStream_t s, uint8_t* xq, float* sx, int block_m,
+                     size_t workspace_bytes, hipStream_t s, uint8_t* xq, float* sx, TileRows tile_rows,
                      int32_t* perm, int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                      int32_t* chunk_counts, int32_t* gemm_cnt, int n_gemm_cnt);
-int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, int block_m, const int32_t* bc,
+int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, TileRows tile_rows, const int32_t* bc,
                              int32_t* perm, int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                              hipStream_t s, int32_t* zero, int nzero);
 extern "C" size_t moe_mi355x_route_workspace_bytes(int T, int H, int E);
@@ -178,7 +178,6 @@ struct ExpertsWs {
   int32_t* bucket; // 16-row tiles: expert buckets [E, T] of pair indices
   size_t total;
   int block_m;
-  int tile_rows;  // rows per tile of the tile list
   int max_tiles;
 };
 
@@ -186,7 +185,6 @@ ExpertsWs carve_experts(void* base, int T, int H, int I, int E, int k) {
   ExpertsWs w{};
   const int S = T * k;
   w.block_m = moe_gemm_block_m(S, E, H, I);
-  w.tile_rows = moe_tile_rows(w.block_m, moe_exact_accum(H));  // block_m at least, so max_tiles holds them
   w.max_tiles = moe_mi355x_align_max_tiles(S, E, w.block_m);
   WsCarver c(base);
   w.xq = c.take<uint8_t>((size_t)T * H);
@@ -229,8 +227,9 @@ int launch_experts(const void* x, const void* ids, int id_bytes, const void* wei
   const int S = T * k;
   int rc;
   if (!prepared) {
-    rc = moe_launch_align(ids, id_bytes, S, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
-                          w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt, x, T, H, w.xq, w.sx);
+    rc = moe_launch_align(ids, id_bytes, S, E, moe_tile_rows(w.block_m, moe_exact_accum(H), H, I), w.perm, w.counts,
+                          w.offsets, w.tiles, w.n_tiles, w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt, x, T, H,
+                          w.xq, w.sx);
     if (rc) return rc;
   }
   // the hand-offs pay on 16-row tiles (batches up to 8 pairs per expert): fewer launches outweigh
@@ -382,16 +381,17 @@ int block_impl(const void* x, const void* w_router, int T, int H, int I, int E, 
   // GEMM), and one launch finishes the sort
   const bool fused = moe_route_can_fuse_align(T, E, k);
   const bool counted = !fused && w.align_ws_bytes > 0;
+  const TileRows tile_rows = moe_tile_rows(w.block_m, moe_exact_accum(H), H, I);
   int rc = moe_launch_route(x, w_router, T, H, E, k, renorm, lg, id_out, idb, wt, b.route_ws, b.route_bytes, s,
-                            w.xq, w.sx, w.tile_rows, fused ? w.perm : nullptr, w.counts, w.offsets, w.tiles,
+                            w.xq, w.sx, tile_rows, fused ? w.perm : nullptr, w.counts, w.offsets, w.tiles,
                             w.n_tiles, counted ? (int32_t*)w.align_ws : nullptr, w.cnt, w.n_cnt);
   if (rc) return rc;
   if (counted) {
-    rc = moe_launch_align_counted(id_out, idb, T * k, E, w.tile_rows, (const int32_t*)w.align_ws, w.perm, w.counts,
+    rc = moe_launch_align_counted(id_out, idb, T * k, E, tile_rows, (const int32_t*)w.align_ws, w.perm, w.counts,
                                   w.offsets, w.tiles, w.n_tiles, s, w.cnt, w.n_cnt);
     if (rc) return rc;
   } else if (!fused) {
-    rc = moe_launch_align(id_out, idb, T * k, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
+    rc = moe_launch_align(id_out, idb, T * k, E, tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
                           w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt);
     if (rc) return rc;
   }
@@ -407,6 +407,13 @@ extern "C" long long moe_mi355x_block_numerics_key(int T, int H, int I, int E, i
   if (!experts_args_ok(T, H, I, E, k, 4) || T == 0) return 0;
   const int bm = fp8 ? moe_gemm_block_m(T * k, E, H, I) : moe_bf16_block_m(T * k, E, H, I);
   return ((long long)moe_route_numerics_key(T, H, E, fp8 != 0) << 16) | bm;
+}
+
+extern "C" int moe_mi355x_experts_tile_rows(int T, int H, int I, int E, int k, int fp8, int tiles_128) {
+  if (!experts_args_ok(T, H, I, E, k, 4) || T == 0) return 0;
+  const int bm = fp8 ? moe_gemm_block_m(T * k, E, H, I) : moe_bf16_block_m(T * k, E, H, I);
+  const TileRows tr = moe_tile_rows(bm, fp8 && moe_exact_accum(H), H, I);
+  return tr.low_tiles > 0 ? moe_pick_rows(tr, tiles_128) : tr.rows;
 }
 
 extern "C" int moe_mi355x_block_fp8(const void* x, const void* w_router, int T, int H, int I, int E, int k,

@@ -20,9 +20,9 @@ int moe_launch_combine(const uint16_t* pairs, const void* ids, int id_bytes, con
                        int E, const uint16_t* residual, uint16_t* out, hipStream_t s);
 int moe_launch_route(const void* x, const void* w_router, int T, int H, int E, int k, int renorm, void* logits,
                      void* ids, int id_bytes, void* weights, void* workspace, size_t workspace_bytes, hipStream_t s,
-                     uint8_t* xq, float* sx, int block_m, int32_t* perm, int32_t* counts, int32_t* offsets,
+                     uint8_t* xq, float* sx, TileRows tile_rows, int32_t* perm, int32_t* counts, int32_t* offsets,
                      int32_t* tiles, int32_t* n_tiles, int32_t* chunk_counts, int32_t* gemm_cnt, int n_gemm_cnt);
-int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, int block_m, const int32_t* bc,
+int moe_launch_align_counted(const void* ids, int id_bytes, int S, int E, TileRows tile_rows, const int32_t* bc,
                              int32_t* perm, int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                              hipStream_t s, int32_t* zero, int nzero);
 bool moe_route_can_fuse_align(int T, int E, int k);
@@ -48,7 +48,6 @@ struct Bf16Ws {
   int32_t* bucket;  // 16-row tiles: expert buckets [E, T] of pair indices
   size_t total;
   int block_m;
-  int tile_rows;  // rows per tile of the tile list
   int max_tiles;
 };
 
@@ -56,7 +55,6 @@ Bf16Ws carve_bf16(void* base, int T, int H, int I, int E, int k) {
   Bf16Ws w{};
   const int S = T * k;
   w.block_m = moe_bf16_block_m(S, E, H, I);
-  w.tile_rows = moe_tile_rows(w.block_m, false);  // block_m at least, so max_tiles holds them
   w.max_tiles = moe_mi355x_align_max_tiles(S, E, w.block_m);
   WsCarver c(base);
   w.perm = c.take<int32_t>(S);
@@ -144,8 +142,8 @@ extern "C" int moe_mi355x_experts_bf16(const void* x, const void* ids, int id_by
   const Bf16Ws w = carve_bf16(workspace, T, H, I, E, k);
   MOE_RETURN_IF(!workspace || workspace_bytes < w.total, MOE_ERR_WORKSPACE);
   hipStream_t s = (hipStream_t)stream;
-  const int rc = moe_launch_align(ids, id_bytes, T * k, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles,
-                                  w.n_tiles, w.align_ws, w.align_ws_bytes, s);
+  const int rc = moe_launch_align(ids, id_bytes, T * k, E, moe_tile_rows(w.block_m, false, H, I), w.perm, w.counts,
+                                  w.offsets, w.tiles, w.n_tiles, w.align_ws, w.align_ws_bytes, s);
   if (rc) return rc;
   return bf16_experts_after_align(x, ids, id_bytes, weights, T, H, I, E, k, w13, w2, out, w, s);
 }
@@ -189,15 +187,16 @@ extern "C" int moe_mi355x_block_bf16(const void* x, const void* w_router, int T,
   // for decode batches, in its own launch(es) above
   const bool fused = moe_route_can_fuse_align(T, E, k);
   const bool counted = !fused && w.align_ws_bytes > 0;
+  const TileRows tile_rows = moe_tile_rows(w.block_m, false, H, I);
   int rc = moe_launch_route(x, w_router, T, H, E, k, renorm, lg, id_out, idb, wt, b.route_ws, b.route_bytes, s,
-                            nullptr, nullptr, w.tile_rows, fused ? w.perm : nullptr, w.counts, w.offsets, w.tiles,
+                            nullptr, nullptr, tile_rows, fused ? w.perm : nullptr, w.counts, w.offsets, w.tiles,
                             w.n_tiles, counted ? (int32_t*)w.align_ws : nullptr, w.cnt, w.n_cnt);
   if (rc) return rc;
   if (counted) {
-    rc = moe_launch_align_counted(id_out, idb, T * k, E, w.tile_rows, (const int32_t*)w.align_ws, w.perm, w.counts,
+    rc = moe_launch_align_counted(id_out, idb, T * k, E, tile_rows, (const int32_t*)w.align_ws, w.perm, w.counts,
                                   w.offsets, w.tiles, w.n_tiles, s, w.cnt, w.n_cnt);
   } else if (!fused) {
-    rc = moe_launch_align(id_out, idb, T * k, E, w.tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
+    rc = moe_launch_align(id_out, idb, T * k, E, tile_rows, w.perm, w.counts, w.offsets, w.tiles, w.n_tiles,
                           w.align_ws, w.align_ws_bytes, s, w.cnt, w.n_cnt);
   }
   if (rc) return rc;

@@ -177,22 +177,10 @@ __device__ __forceinline__ void pf_store_pairs(Acc& acc, const int* s_pairs, con
   }
 }
 
-int device_cu_count() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-      cus = n;
-    else
-      cus = 256;
-  }
-  return cus;
-}
-
 // One persistent workgroup per CU, in whole rounds of the eight XCDs, at most one per work item.
 unsigned pf_grid(const PrefillArgs& a, int max_tiles) {
   const long max_items = (long)max_tiles * a.n_nblk;
-  long grid = device_cu_count();
+  long grid = moe_cu_count();
   if (grid > max_items) grid = max_items;
   grid = (grid + 7) / 8 * 8;
   return (unsigned)(grid < 8 ? 8 : grid);

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const float* __restri
   }
   if (ecnt == nullptr) return;  // kernel-uniform
   __shared__ int s_last;
-  __shared__ int s_cnt[kBuckets], s_off[kBuckets], s_toff[kBuckets];
+  __shared__ int s_cnt[kBuckets], s_off[kBuckets], s_toff[kBuckets], s_rows;
   // every wave's count atomics have returned (their ranks addressed the bucket stores): the
   // workgroup's counts are performed; its other stores (bucket entries, ids, weights) carry no
   // release, so they are read only by later launches (the decode GEMMs), which stream order
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const float* __restri
   if (!s_last) return;
   for (int e = threadIdx.x; e < E; e += blockDim.x) s_cnt[e] = __hip_atomic_load(ecnt + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  scan_counts(s_cnt, E, 16, s_off, s_toff);
+  scan_counts(s_cnt, E, {16, 16, 0}, s_off, s_toff, &s_rows);
   __syncthreads();
   for (int e = threadIdx.x; e <= E; e += blockDim.x) {
     if (e == E) {
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(kChunk) void topk_align_kernel(const float* __restr
                                                             int E, int k, int renorm,
                                                             uint16_t* __restrict__ logits_out, void* ids,
                                                             int id_bytes, uint16_t* __restrict__ weights,
-                                                            int block_m, int32_t* perm, int32_t* counts,
+                                                            TileRows tile_rows, int32_t* perm, int32_t* counts,
                                                             int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                                                             int32_t* gemm_cnt, int n_gemm_cnt) {
   zero_counters(gemm_cnt, n_gemm_cnt);  // the grouped GEMMs' hand-off counters
@@ -298,6 +298,7 @@ __global__ __launch_bounds__(kChunk) void topk_align_kernel(const float* __restr
   __shared__ int s_cnt[kBuckets];
   __shared__ int s_off[kBuckets];
   __shared__ int s_toff[kBuckets];
+  __shared__ int s_rows;
   __shared__ int s_wcnt[kWaves][kBuckets];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int TE = T * E;
@@ -327,9 +328,9 @@ __global__ __launch_bounds__(kChunk) void topk_align_kernel(const float* __restr
   const int S = T * k;
   for (int i = threadIdx.x; i < S; i += blockDim.x) atomicAdd(&s_cnt[s_ids[i]], 1);
   __syncthreads();
-  scan_counts(s_cnt, E, block_m, s_off, s_toff);
+  scan_counts(s_cnt, E, tile_rows, s_off, s_toff, &s_rows);
   __syncthreads();
-  emit_meta(s_cnt, s_off, s_toff, E, block_m, counts, offsets, tiles, n_tiles);
+  emit_meta(s_cnt, s_off, s_toff, E, s_rows, counts, offsets, tiles, n_tiles);
   for (int c0 = 0; c0 < S; c0 += kChunk) scatter_chunk(s_ids, 4, S, E, c0, s_off, s_wcnt, perm);
 }
 
@@ -427,7 +428,7 @@ int moe_launch_router_gemm(const void* x, const void* w_router, int T, int H, in
 // sort run fused in one workgroup and write the align outputs too.
 int moe_launch_route(const void* x, const void* w_router, int T, int H, int E, int k, int renorm,
                      void* logits, void* ids, int id_bytes, void* weights, void* workspace,
-                     size_t workspace_bytes, hipStream_t s, uint8_t* xq, float* sx, int block_m,
+                     size_t workspace_bytes, hipStream_t s, uint8_t* xq, float* sx, TileRows tile_rows,
                      int32_t* perm, int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles,
                      int32_t* chunk_counts, int32_t* gemm_cnt, int n_gemm_cnt) {
   if (T == 0) return MOE_OK;
@@ -443,7 +444,7 @@ int moe_launch_route(const void* x, const void* w_router, int T, int H, int E, i
   float* part = (float*)workspace;
   if (perm != nullptr) {
     MOE_LAUNCH(MOE_PROF_TOPK, s, topk_align_kernel, dim3(1), dim3(kChunk), 0, s, part, ks_eff, T, E, k, renorm,
-               (uint16_t*)logits, ids, id_bytes, (uint16_t*)weights, block_m, perm, counts, offsets, tiles,
+               (uint16_t*)logits, ids, id_bytes, (uint16_t*)weights, tile_rows, perm, counts, offsets, tiles,
                n_tiles, gemm_cnt, n_gemm_cnt);
   } else {
     MOE_LAUNCH(MOE_PROF_TOPK, s, topk_softmax_kernel, dim3((T + 3) / 4), dim3(256), 0, s, part, ks_eff,
@@ -478,7 +479,7 @@ extern "C" int moe_mi355x_route(const void* x, const void* w_router, int T, int 
   MOE_RETURN_IF(!x || !w_router || !ids || !weights, MOE_ERR_INVALID_ARG);
   MOE_RETURN_IF(!moe_aligned16(x) || !moe_aligned16(w_router), MOE_ERR_ALIGNMENT);
   return moe_launch_route(x, w_router, T, H, E, k, renorm, logits, ids, id_bytes, weights, workspace,
-                          workspace_bytes, (hipStream_t)stream, nullptr, nullptr, 0, nullptr, nullptr, nullptr,
+                          workspace_bytes, (hipStream_t)stream, nullptr, nullptr, TileRows{}, nullptr, nullptr, nullptr,
                           nullptr, nullptr, nullptr, nullptr, 0);
 }
 

@@ -1,6 +1,6 @@
 """The combine's forms, and the LDS-tiled grouped GEMMs at the edges of their tiles: experts whose row counts lie around the
-16-row fragments, the two wave groups' shares and the 192- and 144-row tiles, with K loops of 4 and 5
-blocks and with rows of a multiple of 4 KB."""
+16-row fragments, the two wave groups' shares and the 128-, 144- and 192-row tiles, with K loops of 4 and
+5 blocks and with rows of a multiple of 4 KB."""
 
 from __future__ import annotations
 
@@ -22,40 +22,58 @@ def pairs_of(rng, rows):
     return rng.permutation(ids)[:, None]
 
 
-@pytest.mark.parametrize("kind,H,I,rows", [
-    ("fp8", 512, 512, ROWS),                      # 4 K blocks
-    ("fp8", 1024, 640, ROWS),                     # 5 K blocks in the down GEMM
-    ("fp8", 512, 4096, [145, 0, 17, 400]),        # the down GEMM's rows are 4 KB
-    ("fp8", 2304, 512, [144, 1, 145, 81, 300]),   # exact accumulation, 18 K blocks
-    ("fp8", 4096, 512, ROWS),                     # exact, gate_up's rows are 4 KB
-    ("bf16", 256, 256, ROWS),                     # 4 K blocks
-    ("bf16", 512, 384, ROWS),                     # 6 K blocks in the down GEMM
-    ("bf16", 2048, 256, ROWS),                    # gate_up's rows are 4 KB
-    ("bf16", 256, 2048, [193, 0, 17, 192, 300]),  # the down GEMM's rows are 4 KB
+# (repeat: experts rows, rows, .. that many times over, with the same weights each time)
+@pytest.mark.parametrize("kind,H,I,rows,repeat", [
+    ("fp8", 512, 512, ROWS, 1),                      # 4 K blocks
+    ("fp8", 1024, 640, ROWS, 1),                     # 5 K blocks in the down GEMM
+    ("fp8", 512, 4096, [145, 0, 17, 400], 1),        # the down GEMM's rows are 4 KB
+    ("fp8", 512, 1024, ROWS, 6),                     # 4 K blocks in gate_up, four and more items a workgroup
+    ("fp8", 2048, 512, ROWS, 6),                     # the same in the down GEMM
+    ("fp8", 2304, 512, [144, 1, 145, 81, 300], 1),   # exact accumulation, 18 K blocks
+    ("fp8", 4096, 512, ROWS, 1),                     # exact, gate_up's rows are 4 KB
+    ("fp8", 2304, 512, ROWS, 6),                     # exact, 4 K blocks in the down GEMM, its items as above
+    ("bf16", 256, 256, ROWS, 1),                     # 4 K blocks
+    ("bf16", 512, 384, ROWS, 1),                     # 6 K blocks in the down GEMM
+    ("bf16", 2048, 256, ROWS, 1),                    # gate_up's rows are 4 KB
+    ("bf16", 256, 2048, [193, 0, 17, 192, 300], 1),  # the down GEMM's rows are 4 KB
+    ("bf16", 256, 1024, ROWS, 6),                    # 4 K blocks in gate_up, four and more items a workgroup
+    ("bf16", 2048, 256, ROWS, 6),                    # the same in the down GEMM
 ])
-def test_tile_edges(pkg, dev, kind, H, I, rows):
+def test_tile_edges(pkg, dev, kind, H, I, rows, repeat):
+    """Few experts take 128-row tiles (or 144 for exact sums) and at most one or two work items per workgroup;
+    with many experts the tiles have 192 rows, and a workgroup goes from item to item with other row counts."""
     rng = np.random.default_rng(H + I + len(rows))
-    E, ids = len(rows), pairs_of(rng, rows)
+    E0, E, ids = len(rows), len(rows) * repeat, pairs_of(rng, rows * repeat)
     T = len(ids)
-    assert int(pkg._lib.load().moe_mi355x_block_numerics_key(T, H, I, E, 1, int(kind == "fp8"))) & 0xFFFF == 128
+    fp8, exact = int(kind == "fp8"), kind == "fp8" and H > 2048
+    lib = pkg._lib.load()
+    assert int(lib.moe_mi355x_block_numerics_key(T, H, I, E, 1, fp8)) & 0xFFFF == 128
+
+    def tiles(height):
+        return sum(-(-r // height) for r in rows) * repeat
+
+    height = lib.moe_mi355x_experts_tile_rows(T, H, I, E, 1, fp8, tiles(128))
+    assert height == (144 if exact else 128 if repeat == 1 else 192)
+    if repeat > 1:  # more than three rounds of the persistent grid
+        assert tiles(height) * max(I // 128, H // 256) > 3 * torch.cuda.get_device_properties(dev).multi_processor_count
     x = orc.gen_normal_bf16(rng, (T, H))
     w = orc.round_bf16(rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32))
-    w13 = orc.gen_normal_bf16(rng, (E, 2 * I, H), 0.02)
-    w2 = orc.gen_normal_bf16(rng, (E, H, I), 0.02)
-    if kind == "fp8":
+    w13 = orc.gen_normal_bf16(rng, (E0, 2 * I, H), 0.02)
+    w2 = orc.gen_normal_bf16(rng, (E0, H, I), 0.02)
+    if fp8:
         (q13, s13), (q2, s2) = orc.quantize_weight_fp8(w13), orc.quantize_weight_fp8(w2)
-        ref = orc.experts_fp8(x, ids, w, q13, s13, q2, s2)
-        wd = (to_f8(q13, dev), to_dev(s13, dev), to_f8(q2, dev), to_dev(s2, dev))
+        ref = orc.experts_fp8(x, ids % E0, w, q13, s13, q2, s2)
+        wd = (to_f8(np.tile(q13, (repeat, 1, 1)), dev), to_dev(np.tile(s13, (repeat, 1, 1)), dev),
+              to_f8(np.tile(q2, (repeat, 1, 1)), dev), to_dev(np.tile(s2, (repeat, 1, 1)), dev))
         run = pkg.experts_fp8
     else:
-        ref = orc.experts_bf16(x, ids, w, w13, w2, acc=np.float32)
-        wd = (to_bf16(w13, dev), to_bf16(w2, dev))
+        ref = orc.experts_bf16(x, ids % E0, w, w13, w2, acc=np.float32)
+        wd = (to_bf16(w13, dev).repeat(repeat, 1, 1), to_bf16(w2, dev).repeat(repeat, 1, 1))
         run = pkg.experts_bf16
     out = run(to_bf16(x, dev), to_dev(ids, dev), to_bf16(w, dev), *wd)
     max_abs, mean_rel = errors(np_f32(out), ref)
     assert max_abs <= TOL_MAX_ABS and mean_rel <= TOL_MEAN_REL, (max_abs, mean_rel)
-    # a row's sums are taken in an order that only its expert decides: in another place of the tiles it
-    # gives the same bits
+    # a row's sums depend on its expert's weights alone: in another place of the tiles it gives the same bits
     p = rng.permutation(T)
     moved = run(to_bf16(x[p], dev), to_dev(ids[p], dev), to_bf16(w[p], dev), *wd)
     assert torch.equal(moved, out[torch.from_numpy(p).to(dev)])

@@ -28,3 +28,27 @@ int main() {
     subprocess.run(["g++", "-std=c++17", "-I", CSRC, str(src), "-o", str(exe)], check=True)
     read = [int(v) for v in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
     assert read == list(range(rows))
+
+
+def tiles_of(rows, height):
+    return sum(-(-r // height) for r in rows)
+
+
+@pytest.mark.parametrize("fp8,H,I,rows,height", [
+    (1, 2048, 768, [144] * 16, 128),  # 32 tiles of 128 rows x 8 column blocks: a CU for each item
+    (0, 2048, 768, [144] * 16, 128),
+    (1, 2048, 768, [144] * 17, 192),
+    (0, 2048, 768, [144] * 17, 192),
+    (1, 2048, 768, [64] * 128, 192),
+    (1, 2048, 768, [3000] + [0] * 15, 128),
+    (1, 512, 512, [129] * 32, 128),   # 64 tiles x 4 column blocks
+    (1, 512, 512, [129] * 33, 192),
+    (1, 4096, 1536, [144] * 4, 144),  # exact accumulation
+    (0, 4096, 1536, [144] * 8, 128),
+    (1, 2048, 768, [8] * 16, 16),     # 8 pairs per expert: streaming tiles
+    (1, 384, 512, [144] * 4, 64),     # H % 256 != 0: as before
+])
+def test_tile_height_by_items(pkg, fp8, H, I, rows, height):
+    """128-row tiles where all their work items run at once on 256 CUs, else the tallest."""
+    lib = pkg._lib.load()
+    assert lib.moe_mi355x_experts_tile_rows(sum(rows), H, I, len(rows), 1, fp8, tiles_of(rows, 128)) == height
