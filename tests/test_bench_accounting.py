@@ -49,8 +49,8 @@ def test_expected_active_experts(T, expected):
 
 
 def test_prefill_path_matches_library_choice():
-    """bench labels a configuration MFMA-bound exactly where the library runs the 128-row
-    prefill GEMM (16-row tiles up to 8 pairs per expert, then 128-row at these shapes)."""
+    """bench labels a configuration MFMA-bound exactly where the library runs the LDS-tiled
+    prefill GEMM (16-row tiles up to 8 pairs per expert, then key 128 at these shapes)."""
     for shape in (bench.S30B, bench.S235B):
         for T in (1, 64, 128, 256, 257, 1024, 4096):
             S = T * bench.K_TOP
@@ -80,7 +80,7 @@ def test_bf16_bytes():
 
 
 def test_prefill_gate_up_bytes():
-    """On the 128-row path gate_up writes the e4m3 codes of h and one fp32 scale per 128 codes."""
+    """On the LDS-tiled path gate_up writes the e4m3 codes of h and one fp32 scale per 128 codes."""
     s = bench.S30B
     S = 4096 * 8
     assert s.gate_up_bytes(128, 4096) == 128 * 3_146_496 + 4096 * 2048 + 4 * 4096 * 16 + S * 768 + 4 * S * 6

@@ -7,9 +7,9 @@ GPU, through the C ABI.
   ulps of the output scale (the
   bf16 MFMA accumulates exactly in fp32; only the order of fp32 additions differs).
 * the block (router + bf16 experts) against the oracle's bf16 grouped chain on the kernel's
-  routing, at every tile height (16-, 32-, 64- and the LDS-tiled 128-row tiles);
-* the 4096-token Zipf-skewed prefill chunk (C3's routing) on bf16 experts, one token of every
-  128-row tile checked;
+  routing, at every tile height (16-, 32- and 64-row and the LDS tiles);
+* the 4096-token Zipf-skewed prefill chunk (C3's routing) on bf16 experts, tokens of every
+  tile checked;
 * a tiny Qwen3-MoE LM swapped with bf16 blocks, and one dispatching its bf16 experts through
   transformers' ``ExpertsInterface`` under the ``"mi355x"`` key, against transformers' own
   ``grouped_mm`` experts on the same GPU.
@@ -64,8 +64,8 @@ def bf16_block_m(pkg, T, H, I, E, k):
                                           (600, 4096, 1536, 16, 8, 128), (40, 512, 256, 4, 2, 128),
                                           (2, 384, 256, 20, 5, 16)])
 def test_bf16_block_matches_oracle(pkg, dev, T, H, I, E, k, bm):
-    """16-row tiles (S <= 8 E; from 2 tokens on the down GEMM combines each token itself), above the 128-row LDS-tiled kernel; where H % 256 != 0, 32-row
-    tiles (S <= 16 E) and 64-row tiles.  128-row cases at the 30B and 235B widths, with 5 K blocks
+    """16-row tiles (S <= 8 E; from 2 tokens on the down GEMM combines each token itself), above the LDS-tiled kernel; where H % 256 != 0, 32-row
+    tiles (S <= 16 E) and 64-row tiles.  LDS-tiled cases at the 30B and 235B widths, with 5 K blocks
     of 128 in the down GEMM's h (I = 640) and with the minimum of 4 bf16 K blocks (I = 256)."""
     assert bf16_block_m(pkg, T, H, I, E, k) == bm
     rng = np.random.default_rng(400 + T + H)
@@ -96,7 +96,7 @@ def test_bf16_block_matches_oracle(pkg, dev, T, H, I, E, k, bm):
 
 def test_bf16_prefill_zipf_every_tile(pkg, dev):
     """C3's routing (4096 tokens, Zipf-skewed: a few hot experts with many tiles, ragged last
-    tiles) on bf16 30B experts, 128-row tiles; the first, the last and a random row of every tile
+    tiles) on bf16 30B experts, LDS tiles; the first, the last and a random row of every tile
     are checked against the oracle's bf16 chain."""
     from tests.test_gpu_configs import tile_stratified_tokens
 
@@ -110,7 +110,8 @@ def test_bf16_prefill_zipf_every_tile(pkg, dev):
     w13 = (torch.randn((E, 2 * I, H), generator=g, device=dev) * 0.02).to(torch.bfloat16)
     w2 = (torch.randn((E, H, I), generator=g, device=dev) * 0.02).to(torch.bfloat16)
     out = pkg.experts_bf16(to_bf16(x, dev), to_dev(ids, dev), to_bf16(w, dev), w13, w2)
-    sub, n_tiles = tile_stratified_tokens(ids, E, 128, rng)
+    sub, n_tiles, rows = tile_stratified_tokens(pkg, ids, H, I, E, 0, rng)
+    assert rows == 192
     assert n_tiles > 200
     ref = orc.experts_bf16(x[sub], ids[sub], w[sub], np_f32(w13), np_f32(w2), acc=np.float32)
     got = np_f32(out)[sub]

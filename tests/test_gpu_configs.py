@@ -5,7 +5,7 @@ reference's golden vectors.
   top-k ids that transformers' ``Qwen3MoeSparseMoeBlock`` wrote on CPU
   (tests/golden/make_golden.py), and the FP8 block on the same inputs against the oracle.
 * C2: decode batches including 128 and 129 tokens, the 8 E pair count where the expert GEMMs
-  switch from 16-row streaming tiles to the 128-row LDS-tiled kernel, and 256 tokens
+  switch from 16-row streaming tiles to the LDS-tiled kernel, and 256 tokens
   (tests/test_gpu_parity.py covers 1, 8, 32, 64, 256).
 * C3: the 4096-token Zipf-skewed prefill chunk, checked on a tile-stratified token sample: the
   first, the last and a random row of every M tile of the expert GEMMs (ragged remainders of the
@@ -42,17 +42,19 @@ def block_m_of(pkg, T, H, I, E, k):
     return int(pkg._lib.load().moe_mi355x_block_numerics_key(T, H, I, E, k, 1)) & 0xFFFF
 
 
-def tile_stratified_tokens(ids, E, block_m, rng):
-    """Tokens owning the first, the last and a random row of every block_m-row tile of the
-    stable expert sort (oracle align + tile_list), so every tile the GEMMs run is checked."""
-    k = ids.shape[1]
+def tile_stratified_tokens(pkg, ids, H, I, E, fp8, rng):
+    """Tokens owning the first, the last and a random row of every tile of the stable expert sort
+    (oracle align + tile_list at the height that the library picks for these counts), so every tile
+    the GEMMs run is checked.  Also the number of tiles and their height."""
+    T, k = ids.shape
     perm, counts, _ = orc.align(ids, E)
     toks = set()
-    tiles = orc.tile_list(counts, block_m)
+    height = pkg._lib.load().moe_mi355x_experts_tile_rows(T, H, I, E, k, fp8, len(orc.tile_list(counts, 128)))
+    tiles = orc.tile_list(counts, height)
     for _, r0, rows in tiles:
         for r in (r0, r0 + rows - 1, r0 + int(rng.integers(rows))):
             toks.add(int(perm[r]) // k)
-    return np.array(sorted(toks)), len(tiles)
+    return np.array(sorted(toks)), len(tiles), height
 
 
 def check_experts(pkg, dev, x, ids, w, weights_dev, weights_np, sub=None):
@@ -144,7 +146,7 @@ def w30b(dev):
 
 @pytest.mark.parametrize("T", [127, 128, 129, 256])
 def test_c2_decode_tile_switch(pkg, dev, w30b, T):
-    """Around S = 8 E = 1024 pairs: 16-row tiles up to 128 tokens, the 128-row LDS-tiled kernel
+    """Around S = 8 E = 1024 pairs: 16-row tiles up to 128 tokens, the LDS-tiled kernel
     from 129 (every token checked)."""
     assert block_m_of(pkg, T, 2048, 768, 128, 8) == (16 if T <= 128 else 128)
     rng = np.random.default_rng(200 + T)
@@ -163,7 +165,8 @@ def test_c3_prefill_zipf_every_tile(pkg, dev, w30b):
     assert np.sort(counts)[::-1][:10].sum() / (T * k) > 0.4  # skewed: a few hot experts
     bm = block_m_of(pkg, T, H, 768, E, k)
     assert bm == 128
-    sub, n_tiles = tile_stratified_tokens(ids, E, bm, rng)
+    sub, n_tiles, rows = tile_stratified_tokens(pkg, ids, H, 768, E, 1, rng)
+    assert rows == 192
     assert n_tiles > 200
     check_experts(pkg, dev, x, ids, w, *w30b, sub=sub)
 
@@ -197,7 +200,8 @@ def test_c4_235b_prefill_2048_every_tile(pkg, dev, w235b):
     ids, w = orc.uniform_routing(rng, T, 128, 8)
     bm = block_m_of(pkg, T, 4096, 1536, 128, 8)
     assert bm == 128
-    sub, n_tiles = tile_stratified_tokens(ids, 128, bm, rng)
+    sub, n_tiles, rows = tile_stratified_tokens(pkg, ids, 4096, 1536, 128, 1, rng)
+    assert rows == 144
     assert n_tiles >= 128
     check_experts(pkg, dev, x, ids, w, *w235b, sub=sub)
 

@@ -227,7 +227,7 @@ def test_compiled_swapped_model_matches_eager(pkg, dev):
 
 
 def test_graphed_bf16_block_across_tile_heights(pkg, dev):
-    """bf16 experts, E = 16, k = 4: 16-row tiles up to 32 tokens, then the LDS-tiled 128-row
+    """bf16 experts, E = 16, k = 4: 16-row tiles up to 32 tokens, then the LDS-tiled
     kernel.  Each tiling gets bucket edges of its own, and every replay equals the eager block bit
     for bit."""
     E, H, I, k = 16, 512, 256, 4
@@ -253,7 +253,7 @@ def test_graphed_bf16_block_across_tile_heights(pkg, dev):
 def test_compiled_bf16_swapped_model_matches_eager(pkg, dev):
     """The same with the default bf16 checkpoint kept in bf16 (torch.ops.moe_mi355x.moe_block_bf16):
     a compiled prefill and decode step of the model equal eager bit for bit, and the swapped block
-    compiled on its own equals eager on an 80-token chunk, which runs the 128-row bf16 tiles.  (The
+    compiled on its own equals eager on an 80-token chunk, which runs the LDS tiles.  (The
     whole model is compared at 10 tokens: at 40 transformers' own compiled attention path already
     differs from eager in the last bits, with FP8 blocks as with bf16 ones.)"""
     from transformers import DynamicCache
@@ -278,7 +278,7 @@ def test_compiled_bf16_swapped_model_matches_eager(pkg, dev):
         want1 = step(nxt, cache_e)
         got1 = compiled(nxt, cache_c)
         assert torch.equal(got1, want1)
-        # 80 tokens x 4 slots > 16 E: the 128-row bf16 tiles
+        # 80 tokens x 4 slots > 16 E: the LDS tiles
         key = pkg._lib.load().moe_mi355x_block_numerics_key(80, 256, 256, 16, 4, 0)
         assert int(key) & 0xFFFF == 128
         x = torch.randn((2, 40, 256), device=dev).to(torch.bfloat16)

@@ -183,7 +183,7 @@ def test_experts_decode_30b(pkg, dev, w30b, T):
 def test_experts_ep_share_30b(pkg, dev, R):
     """One GPU's share of 8-way expert parallelism (bench.py's ep_share entry): 16 local experts at
     the 30B H / I, R received rows with one local expert each (k = 1); 8 rows take the 16-row
-    tiles, 512 rows the 128-row prefill tiles (S > 8 E)."""
+    tiles, 512 rows the LDS tiles (S > 8 E)."""
     E = 16
     rng = np.random.default_rng(20 + R)
     x = orc.gen_normal_bf16(rng, (R, 2048))
@@ -207,7 +207,7 @@ def test_experts_prefill_skewed_30b(pkg, dev, w30b):
 
 @pytest.mark.parametrize("T", [300, 1024])
 def test_experts_prefill_uniform_30b(pkg, dev, w30b, T):
-    """128-row LDS-tiled path (S > 16 E) with ragged last tiles per expert."""
+    """LDS-tiled path (S > 8 E) with ragged last tiles per expert."""
     rng = np.random.default_rng(20 + T)
     x = orc.gen_normal_bf16(rng, (T, 2048))
     ids, w = orc.uniform_routing(rng, T, 128, 8)
@@ -293,7 +293,7 @@ def test_block_30b_routing_paths(pkg, dev, w30b, router30b, T):
     assert max_abs <= TOL_MAX_ABS and mean_rel <= TOL_MEAN_REL
 
 
-@pytest.mark.parametrize("T", [40, 600])  # 16-row decode tiles; 128-row prefill tiles
+@pytest.mark.parametrize("T", [40, 600])  # 16-row decode tiles; LDS tiles
 def test_sentinel_pairs_contribute_zero(pkg, dev, w30b, T):
     """Expert-parallel sentinels (ids outside [0, E), moe.py:405-419) add nothing: the output
     equals, bit for bit, the same routing with those slots' weights set to zero (every pair
@@ -342,10 +342,10 @@ SHAPE_SWEEP = [
     (30, 512, 256, 10, 4),     # 32-row tiles
     (40, 384, 256, 6, 3),      # 64-row tiles (H % 256 != 0)
     (77, 1024, 384, 20, 5),    # 64-row tiles (I < 512)
-    (300, 512, 512, 16, 4),    # 128-row prefill tiles, 4 K blocks per GEMM
-    (257, 1024, 640, 12, 6),   # 128-row prefill tiles, 5 K blocks in the down GEMM
+    (300, 512, 512, 16, 4),    # LDS tiles, 4 K blocks per GEMM
+    (257, 1024, 640, 12, 6),   # LDS tiles, 5 K blocks in the down GEMM
     (24, 256, 4096, 2, 1),     # the largest intermediate size: 32 K blocks in the down GEMM
-    (600, 512, 4096, 4, 2),    # the same on the 128-row prefill tiles
+    (600, 512, 4096, 4, 2),    # the same on the LDS tiles
     (2, 256, 1536, 16, 4),     # routed one-row slots, h quantised in gate_up's hand-off (I > 1024)
     (6, 256, 1536, 32, 4),     # expert buckets, S <= 2 E: h quantised in gate_up's hand-off
     (2, 256, 2048, 16, 4),     # the same two at I = 2048
@@ -357,7 +357,7 @@ SHAPE_SWEEP = [
     (5, 4096, 256, 8, 2),      # H > 2048: exact bf16 MFMAs on widened e4m3, 16-row tiles
     (30, 4096, 256, 10, 4),    # exact, 32-row tiles
     (60, 4096, 256, 10, 4),    # exact, 64-row tiles
-    (300, 4096, 512, 8, 4),    # exact, 128-row prefill tiles
+    (300, 4096, 512, 8, 4),    # exact, LDS tiles
 ]
 
 

@@ -81,13 +81,21 @@ def test_tile_edges(pkg, dev, kind, H, I, rows, repeat):
 
 @pytest.mark.parametrize("k", [1, 8, 12, 16])
 @pytest.mark.parametrize("id_type", [torch.int32, torch.int64])
-@pytest.mark.parametrize("T,H", [(7, 256), (130, 2304)])
-def test_combine_forms(pkg, dev, T, H, k, id_type):
-    """Weights one by one (k % 8 != 0, or rows of 8 at an odd address) and eight at a time, ids of both
+@pytest.mark.parametrize("T,H,I", [
+    (7, 256, 256),     # pair rows that the GEMM has weighted: streaming tiles
+    (130, 2304, 256),  # the same, two column blocks
+    (130, 768, 512),   # LDS tiles, whose pair rows the combine weights: one column block of 96 threads
+    (130, 2304, 512),  # the same, two column blocks (exact accumulation)
+])
+def test_combine_forms(pkg, dev, T, H, I, k, id_type):
+    """Pair rows weighted already (H or I below the LDS tiles' or few pairs), weights one by one (k % 8 != 0,
+    or rows of 8 at an odd address) and eight at a time, one and two passes over the slots, ids of both
     sizes with sentinels on either side of the range (for 64-bit ids also ones whose low word is an
     expert), one and two column blocks with a remainder."""
     rng = np.random.default_rng(T + k)
-    E, I = 16, 256
+    E = 16
+    key = int(pkg._lib.load().moe_mi355x_block_numerics_key(T, H, I, E, k, 1)) & 0xFFFF
+    assert (key == 128) == (I == 512)  # the LDS tiles leave the weights to the combine
     ids = np.argsort(rng.random((T, E)), axis=1)[:, :k].astype(np.int64)
     ids[0, 0], ids[T // 2, -1] = -1, E
     if id_type == torch.int64:
@@ -103,7 +111,9 @@ def test_combine_forms(pkg, dev, T, H, k, id_type):
     out = pkg.experts_fp8(to_bf16(x, dev), di, to_bf16(w, dev), *wd)
     max_abs, mean_rel = errors(np_f32(out), ref)
     assert max_abs <= TOL_MAX_ABS and mean_rel <= TOL_MEAN_REL, (max_abs, mean_rel)
+    # the rows' address alone decides between one by one and eight at a time
     odd = torch.empty(T * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(T, k).copy_(to_bf16(w, dev))
+    assert odd.data_ptr() % 16 == 2
     assert torch.equal(pkg.experts_fp8(to_bf16(x, dev), di, odd, *wd), out)
 
 
