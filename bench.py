@@ -68,7 +68,7 @@ class Shape:
         the fp8 activations and their scales read, the intermediate written: bf16 h, which the
         16-row down GEMM quantises as it loads it where its LDS rows hold I (I <= 1024); else up
         to 2 pairs per expert (S <= 2 E) the launch quantises it itself (e4m3 codes + scales, and
-        its bf16 h round trip between the launch's workgroups is counted too).  On the 128-row
+        its bf16 h round trip between the launch's workgroups is counted too).  On the LDS-tiled
         prefill path the launch writes the e4m3 codes of h and their scales."""
         S = T * K_TOP
         if self.prefill_path(T):  # the LDS-tiled kernel writes the e4m3 codes of h and their scales

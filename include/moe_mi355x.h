@@ -287,6 +287,8 @@ int moe_mi355x_moe_sublayer_fp8(const void* h, const void* h_add, const void* ln
  * waits for them and returns the launch count and summed duration (ms) of one slot:
  *   0 router_gemm  1 topk_softmax  2 quant_act  3 align  4 gemm_gate_up  5 quant_h
  *   6 gemm_down    7 combine   8 linear
+ * The activation quantisation of an FP8 call has no slot of its own: it is part of router_gemm's launch
+ * (blocks) or of align's first one (moe_mi355x_experts_fp8).  quant_act is moe_mi355x_quantize_act_fp8.
  * Enabling (or disabling) clears what was recorded.
  */
 int moe_mi355x_profile_enable(int on);

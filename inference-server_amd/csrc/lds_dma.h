@@ -1,5 +1,5 @@
-// LDS staging helpers of the LDS-tiled grouped GEMMs (gemm_prefill.hip): the swizzled 128-byte LDS row layout, MFMA fragment reads,
-// global -> LDS DMA, wait / barrier and scalar table loads.
+// LDS staging helpers of the LDS-tiled grouped GEMMs (gemm_prefill.hip, gemm_prefill_exact.hip): the swizzled
+// 128-byte LDS row layout, global -> LDS DMA, wait / barrier and scalar table loads.
 #pragma once
 
 #include "common.h"
@@ -13,16 +13,6 @@ namespace moe_lds {
 // SQ_LDS_BANK_CONFLICT; XOR with r & 7 or (r >> 1) & 7 alone costs 8).  The key depends on
 // r & 15 only, so a lane's address within any 16-row group is the same.
 __device__ __forceinline__ int swz_key(int row) { return (row ^ ((row >> 3) & 1)) & 7; }
-__device__ __forceinline__ int swz(int row, int chunk) { return row * 128 + ((chunk ^ swz_key(row)) << 4); }
-
-__device__ __forceinline__ v8i lds_frag(const uint8_t* base, int row, int c0) {
-  const uint4 lo = *(const uint4*)(base + swz(row, c0));
-  const uint4 hi = *(const uint4*)(base + swz(row, c0 + 1));
-  v8i r;
-  r[0] = lo.x; r[1] = lo.y; r[2] = lo.z; r[3] = lo.w;
-  r[4] = hi.x; r[5] = hi.y; r[6] = hi.z; r[7] = hi.w;
-  return r;
-}
 
 #define LDS_AS __attribute__((address_space(3)))
 
