@@ -179,11 +179,12 @@ int moe_mi355x_block_fp8_noalloc(const void* x, const void* w_router, int T, int
 long long moe_mi355x_block_numerics_key(int T, int H, int I, int E, int k, int fp8);
 
 /*
- * Rows per tile of one expert's sorted rows in the expert GEMMs of the FP8 (fp8 != 0) or the bf16
- * entry points, for a routing that cuts into tiles_128 tiles of at most 128 rows (each expert's rows on
- * their own).  No result depends on it.  0 for unsupported shapes.  A query (host only).
+ * Rows per tile in the expert GEMMs of the FP8 (fp8 != 0) or the bf16 entry points, for a routing that
+ * gives expert e counts[e] rows: returns the most that a tile may have, and in rows[e] (both host arrays
+ * of E; rows may be null) what the tiles of expert e have, but for its last.  No result depends on it.
+ * 0 for unsupported shapes and counts.  A query (host only).
  */
-int moe_mi355x_experts_tile_rows(int T, int H, int I, int E, int k, int fp8, int tiles_128);
+int moe_mi355x_experts_tile_rows(int T, int H, int I, int E, int k, int fp8, const int* counts, int* rows);
 
 /*
  * Paged GQA decode attention, one new token per sequence (the attention of a decode step of

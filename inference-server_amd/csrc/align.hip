@@ -57,7 +57,7 @@ __global__ __launch_bounds__(kChunk) void align_single_kernel(const void* ids, i
   __syncthreads();
   scan_counts(s_cnt, E, tile_rows, s_off, s_toff, &s_rows);
   __syncthreads();
-  emit_meta(s_cnt, s_off, s_toff, E, s_rows, counts, offsets, tiles, n_tiles);
+  emit_meta(s_cnt, s_off, s_toff, E, tile_rows, s_rows, counts, offsets, tiles, n_tiles);
   // s_off doubles as the running base from here on; s_off[E] starts the sentinel tail
   for (int c0 = 0; c0 < S; c0 += kChunk) scatter_chunk(ids, id_bytes, S, E, c0, s_off, s_wcnt, perm);
 }
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kChunk) void align_scan_scatter_kernel(const void* 
   __syncthreads();
   scan_counts(s_cnt, E, tile_rows, s_off, s_toff, &s_rows);
   __syncthreads();
-  if (b == 0) emit_meta(s_cnt, s_off, s_toff, E, s_rows, counts, offsets, tiles, n_tiles);
+  if (b == 0) emit_meta(s_cnt, s_off, s_toff, E, tile_rows, s_rows, counts, offsets, tiles, n_tiles);
   for (int e = threadIdx.x; e <= E; e += blockDim.x) s_base[e] += s_off[e];
   __syncthreads();
   scatter_chunk(ids, id_bytes, S, E, b * kChunk, s_base, s_wcnt, perm);
@@ -180,6 +180,6 @@ extern "C" int moe_mi355x_align(const void* ids, int id_bytes, int T, int k, int
   MOE_RETURN_IF(S > (1L << 30), MOE_ERR_INVALID_ARG);
   MOE_RETURN_IF(S > 0 && (!ids || !perm || !tiles), MOE_ERR_INVALID_ARG);
   MOE_RETURN_IF(!moe_aligned16(tiles), MOE_ERR_ALIGNMENT);
-  return moe_launch_align(ids, id_bytes, (int)S, E, {block_m, block_m, 0}, perm, counts, offsets, tiles, n_tiles, workspace,
+  return moe_launch_align(ids, id_bytes, (int)S, E, {block_m}, perm, counts, offsets, tiles, n_tiles, workspace,
                           workspace_bytes, (hipStream_t)stream);
 }

@@ -21,40 +21,48 @@ constexpr int kSingleMaxS = 4096;  // pairs the one-workgroup top-k + sort kerne
 // slots 13.5 -> 7.6 us.
 constexpr int kAlignOneWgMaxS = 2048;
 
-// Picks the rows per tile (s_rows[0]), then exclusive scans of counts and of ceil(count / rows) over
-// experts; wave 0 of the block.
-__device__ void scan_counts(const int* s_cnt, int E, TileRows tr, int* s_off, int* s_toff, int* s_rows) {
+// Exclusive scans of counts and of ceil(count / rows) over experts, and the rows per tile (s_rows[0]);
+// wave 0 of the block.
+__device__ void scan_counts(const int* s_cnt, int E, const TileRows& tr, int* s_off, int* s_toff, int* s_rows) {
   const int lane = threadIdx.x & 63;
   if ((threadIdx.x >> 6) != 0) return;
-  int c[4], t[4], sc = 0, st = 0;
+  constexpr int kLow = kPrefillLowRows, kHigh = moe_prefill_rows(false);  // constants: no division by a variable
+  int c[4], t[4], u[4], sc = 0, st = 0, su = 0;  // u: tiles of kLow rows, where those are a choice
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int e = lane * 4 + q;
     c[q] = e < E ? s_cnt[e] : 0;
-  }
-  int rows = tr.rows;
-  if (tr.low_tiles > 0) {  // kernel-uniform
-    int n = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) n += (c[q] + tr.low - 1) / tr.low;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d, MOE_WAVE);
-    rows = moe_pick_rows(tr, n);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    t[q] = (c[q] + rows - 1) / rows;
     sc += c[q];
-    st += t[q];
   }
-  int ic = sc, it = st;
+  if (tr.pick) {  // kernel-uniform
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      su += u[q] = (c[q] + kLow - 1) / kLow;
+      st += t[q] = (c[q] + kHigh - 1) / kHigh;
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      u[q] = 0;
+      st += t[q] = (c[q] + tr.rows - 1) / tr.rows;
+    }
+  }
+  int ic = sc, it = st, iu = su;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const int oc = __shfl_up(ic, d, MOE_WAVE), ot = __shfl_up(it, d, MOE_WAVE);
+    const int oc = __shfl_up(ic, d, MOE_WAVE), ot = __shfl_up(it, d, MOE_WAVE), ou = __shfl_up(iu, d, MOE_WAVE);
     if (lane >= d) {
       ic += oc;
       it += ot;
+      iu += ou;
     }
+  }
+  const int rows = moe_pick_rows(tr, __builtin_amdgcn_readlane(iu, 63), __builtin_amdgcn_readlane(it, 63));
+  if (tr.pick && rows == kLow) {
+    it = iu;
+    st = su;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) t[q] = u[q];
   }
   int ec = ic - sc, et = it - st;
 #pragma unroll
@@ -81,7 +89,7 @@ __device__ __forceinline__ void zero_counters(int32_t* zero, int n) {
 }
 
 // Writes counts, offsets and the tile list from the scanned LDS arrays.
-__device__ void emit_meta(const int* s_cnt, const int* s_off, const int* s_toff, int E, int rows,
+__device__ void emit_meta(const int* s_cnt, const int* s_off, const int* s_toff, int E, const TileRows& tr, int rows,
                           int32_t* counts, int32_t* offsets, int32_t* tiles, int32_t* n_tiles) {
   for (int e = threadIdx.x; e <= E; e += blockDim.x) {
     offsets[e] = s_off[e];
@@ -92,8 +100,9 @@ __device__ void emit_meta(const int* s_cnt, const int* s_off, const int* s_toff,
     const int c = s_cnt[e];
     counts[e] = c;
     int tix = s_toff[e];
-    for (int r = 0; r < c; r += rows, ++tix) {
-      int4 v = make_int4(e, s_off[e] + r, min(rows, c - r), 0);
+    const int h = moe_expert_rows(tr, c, rows);
+    for (int r = 0; r < c; r += h, ++tix) {
+      int4 v = make_int4(e, s_off[e] + r, min(h, c - r), 0);
       *(int4*)(tiles + 4 * tix) = v;
     }
   }

@@ -82,9 +82,11 @@ __device__ __forceinline__ v4f mfma_e4m3_exact(const v8i& a, const v8i& b) {
 // f8f6f4 MFMA (twice the bf16 rate) is kept there.
 __host__ __device__ inline bool moe_exact_accum(int H) { return H > 2048; }
 
-// Rows per tile of the expert sort's tile list: `rows`, or `low` where those give at most low_tiles tiles.
+// Rows per tile of the expert sort's tile list.
 struct TileRows {
-  int rows, low, low_tiles;
+  int rows;
+  bool pick, even;    // or kPrefillLowRows where pf_cut_low says so; an expert's tiles equally high
+  int nb1, nb2, cus;  // pick: column blocks per tile of the two GEMMs, CUs
 };
 
 // CUs of the current device (the first call's: all GPUs of a node are alike).
@@ -102,13 +104,18 @@ inline int moe_cu_count() {
 // ... for tile height block_m: the height that picks a GEMM, of which 128 names the LDS-tiled ones of the
 // larger batches.  No tile is lower than block_m (unless its expert ends), so block_m bounds their number.
 inline TileRows moe_tile_rows(int block_m, bool exact, int H, int I) {
-  if (block_m != 128) return {block_m, block_m, 0};
-  return {moe_prefill_rows(exact), kPrefillLowRows, moe_prefill_low_tiles(exact, H, I, moe_cu_count())};
+  if (block_m != 128) return {block_m};
+  return {moe_prefill_rows(exact), !exact, true, I / 128, H / 256, moe_cu_count()};
 }
 
-// The rows of a list that has n_low tiles of tr.low rows.
-__host__ __device__ inline int moe_pick_rows(const TileRows& tr, int n_low) {
-  return n_low <= tr.low_tiles ? tr.low : tr.rows;
+// The rows of a list that would have n_low tiles of kPrefillLowRows rows or n tiles of tr.rows.
+__host__ __device__ inline int moe_pick_rows(const TileRows& tr, int n_low, int n) {
+  return tr.pick && pf_cut_low(n_low, n, tr.nb1, tr.nb2, tr.cus) ? kPrefillLowRows : tr.rows;
+}
+
+// Rows per tile of an expert with n rows in a list of `rows` rows per tile.
+__host__ __device__ inline int moe_expert_rows(const TileRows& tr, int n, int rows) {
+  return tr.even ? pf_even_rows(n, rows) : rows;
 }
 
 // silu(gate) * up on bf16 values, in the reference's rounding order: the grouped GEMM

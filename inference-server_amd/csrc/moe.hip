@@ -409,11 +409,20 @@ extern "C" long long moe_mi355x_block_numerics_key(int T, int H, int I, int E, i
   return ((long long)moe_route_numerics_key(T, H, E, fp8 != 0) << 16) | bm;
 }
 
-extern "C" int moe_mi355x_experts_tile_rows(int T, int H, int I, int E, int k, int fp8, int tiles_128) {
-  if (!experts_args_ok(T, H, I, E, k, 4) || T == 0) return 0;
+extern "C" int moe_mi355x_experts_tile_rows(int T, int H, int I, int E, int k, int fp8, const int* counts,
+                                            int* rows) {
+  if (!experts_args_ok(T, H, I, E, k, 4) || T == 0 || !counts) return 0;
   const int bm = fp8 ? moe_gemm_block_m(T * k, E, H, I) : moe_bf16_block_m(T * k, E, H, I);
   const TileRows tr = moe_tile_rows(bm, fp8 && moe_exact_accum(H), H, I);
-  return tr.low_tiles > 0 ? moe_pick_rows(tr, tiles_128) : tr.rows;
+  int n_low = 0, n = 0;
+  for (int e = 0; e < E; ++e) {
+    if (counts[e] < 0 || counts[e] > T * k) return 0;
+    n_low += (counts[e] + kPrefillLowRows - 1) / kPrefillLowRows;
+    n += (counts[e] + tr.rows - 1) / tr.rows;
+  }
+  const int most = moe_pick_rows(tr, n_low, n);
+  for (int e = 0; rows && e < E; ++e) rows[e] = moe_expert_rows(tr, counts[e], most);
+  return most;
 }
 
 extern "C" int moe_mi355x_block_fp8(const void* x, const void* w_router, int T, int H, int I, int E, int k,

@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const float* __restri
   if (!s_last) return;
   for (int e = threadIdx.x; e < E; e += blockDim.x) s_cnt[e] = __hip_atomic_load(ecnt + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  scan_counts(s_cnt, E, {16, 16, 0}, s_off, s_toff, &s_rows);
+  scan_counts(s_cnt, E, {16}, s_off, s_toff, &s_rows);
   __syncthreads();
   for (int e = threadIdx.x; e <= E; e += blockDim.x) {
     if (e == E) {
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(kChunk) void topk_align_kernel(const float* __restr
   __syncthreads();
   scan_counts(s_cnt, E, tile_rows, s_off, s_toff, &s_rows);
   __syncthreads();
-  emit_meta(s_cnt, s_off, s_toff, E, s_rows, counts, offsets, tiles, n_tiles);
+  emit_meta(s_cnt, s_off, s_toff, E, tile_rows, s_rows, counts, offsets, tiles, n_tiles);
   for (int c0 = 0; c0 < S; c0 += kChunk) scatter_chunk(s_ids, 4, S, E, c0, s_off, s_wcnt, perm);
 }
 

@@ -56,3 +56,10 @@ def gpu_weights(E, H, I, dev, seed=0, std=0.02):
     q2, s2 = pkg.quantize_weight_fp8(w2)
     del w13, w2
     return q13, s13, q2, s2
+
+
+def tile_rows(pkg, counts, T, H, I, k, fp8):
+    """Most rows per tile, and each expert's, as the library cuts them."""
+    c, rows = np.asarray(counts, dtype=np.int32), np.zeros(len(counts), dtype=np.int32)
+    most = pkg._lib.load().moe_mi355x_experts_tile_rows(T, H, I, len(c), k, fp8, c.ctypes.data, rows.ctypes.data)
+    return most, rows

@@ -28,7 +28,7 @@ import torch
 
 from oracle import moe_oracle as orc
 from tests.helpers import (TOL_MAX_ABS, TOL_MEAN_REL, bf16_ulp_diff, errors, f8_codes, gpu_weights, np_f32,
-                           to_bf16, to_dev)
+                           tile_rows, to_bf16, to_dev)
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 sys.path.insert(0, GOLDEN)
@@ -44,17 +44,19 @@ def block_m_of(pkg, T, H, I, E, k):
 
 def tile_stratified_tokens(pkg, ids, H, I, E, fp8, rng):
     """Tokens owning the first, the last and a random row of every tile of the stable expert sort
-    (oracle align + tile_list at the height that the library picks for these counts), so every tile
-    the GEMMs run is checked.  Also the number of tiles and their height."""
+    (oracle align, cut as the library cuts these counts), so every tile the GEMMs run is checked.
+    Also the number of tiles and the most rows of one."""
     T, k = ids.shape
-    perm, counts, _ = orc.align(ids, E)
-    toks = set()
-    height = pkg._lib.load().moe_mi355x_experts_tile_rows(T, H, I, E, k, fp8, len(orc.tile_list(counts, 128)))
-    tiles = orc.tile_list(counts, height)
-    for _, r0, rows in tiles:
-        for r in (r0, r0 + rows - 1, r0 + int(rng.integers(rows))):
-            toks.add(int(perm[r]) // k)
-    return np.array(sorted(toks)), len(tiles), height
+    perm, counts, offsets = orc.align(ids, E)
+    toks, n_tiles = set(), 0
+    height, tile = tile_rows(pkg, counts, T, H, I, k, fp8)
+    for e in range(E):
+        for r0 in range(0, int(counts[e]), int(tile[e])):
+            rows = min(int(tile[e]), int(counts[e]) - r0)
+            n_tiles += 1
+            for r in (r0, r0 + rows - 1, r0 + int(rng.integers(rows))):
+                toks.add(int(perm[int(offsets[e]) + r]) // k)
+    return np.array(sorted(toks)), n_tiles, height
 
 
 def check_experts(pkg, dev, x, ids, w, weights_dev, weights_np, sub=None):

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import moe_oracle as orc
-from tests.helpers import TOL_MAX_ABS, TOL_MEAN_REL, errors, np_f32, to_bf16, to_dev, to_f8
+from tests.helpers import TOL_MAX_ABS, TOL_MEAN_REL, errors, np_f32, tile_rows, to_bf16, to_dev, to_f8
 
 pytestmark = pytest.mark.gpu
 
@@ -49,13 +49,11 @@ def test_tile_edges(pkg, dev, kind, H, I, rows, repeat):
     lib = pkg._lib.load()
     assert int(lib.moe_mi355x_block_numerics_key(T, H, I, E, 1, fp8)) & 0xFFFF == 128
 
-    def tiles(height):
-        return sum(-(-r // height) for r in rows) * repeat
-
-    height = lib.moe_mi355x_experts_tile_rows(T, H, I, E, 1, fp8, tiles(128))
+    height, tile = tile_rows(pkg, rows * repeat, T, H, I, 1, fp8)
     assert height == (144 if exact else 128 if repeat == 1 else 192)
     if repeat > 1:  # more than three rounds of the persistent grid
-        assert tiles(height) * max(I // 128, H // 256) > 3 * torch.cuda.get_device_properties(dev).multi_processor_count
+        tiles = sum(-(-r // h) for r, h in zip(rows * repeat, tile.tolist()))
+        assert tiles * max(I // 128, H // 256) > 3 * torch.cuda.get_device_properties(dev).multi_processor_count
     x = orc.gen_normal_bf16(rng, (T, H))
     w = orc.round_bf16(rng.uniform(0.2, 1.0, (T, 1)).astype(np.float32))
     w13 = orc.gen_normal_bf16(rng, (E0, 2 * I, H), 0.02)

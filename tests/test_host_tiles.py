@@ -7,6 +7,8 @@ import subprocess
 
 import pytest
 
+from tests.helpers import tile_rows
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "inference-server_amd", "csrc")
 
 
@@ -30,16 +32,18 @@ int main() {
     assert read == list(range(rows))
 
 
-def tiles_of(rows, height):
-    return sum(-(-r // height) for r in rows)
-
-
 @pytest.mark.parametrize("fp8,H,I,rows,height", [
     (1, 2048, 768, [144] * 16, 128),  # 32 tiles of 128 rows x 8 column blocks: a CU for each item
     (0, 2048, 768, [144] * 16, 128),
-    (1, 2048, 768, [144] * 17, 192),
+    (1, 2048, 768, [144] * 17, 192),  # one round of 192-row tiles, two of 128-row ones
     (0, 2048, 768, [144] * 17, 192),
-    (1, 2048, 768, [64] * 128, 192),
+    (1, 2048, 768, [190] * 8 + [210] * 24, 128),  # 64 and 56 tiles, two rounds of either
+    (0, 2048, 768, [190] * 8 + [210] * 24, 128),
+    (1, 2048, 768, [430] * 16, 128),  # 64 and 48 tiles, two rounds of either
+    (0, 2048, 768, [430] * 16, 128),
+    (1, 2048, 768, [300] * 16, 192),  # 48 and 32 tiles: two rounds and one
+    (1, 2048, 768, [150] * 128, 192),
+    (1, 2048, 768, [64] * 128, 128),  # one tile each, whatever the height
     (1, 2048, 768, [3000] + [0] * 15, 128),
     (1, 512, 512, [129] * 32, 128),   # 64 tiles x 4 column blocks
     (1, 512, 512, [129] * 33, 192),
@@ -49,6 +53,22 @@ def tiles_of(rows, height):
     (1, 384, 512, [144] * 4, 64),     # H % 256 != 0: as before
 ])
 def test_tile_height_by_items(pkg, fp8, H, I, rows, height):
-    """128-row tiles where all their work items run at once on 256 CUs, else the tallest."""
-    lib = pkg._lib.load()
-    assert lib.moe_mi355x_experts_tile_rows(sum(rows), H, I, len(rows), 1, fp8, tiles_of(rows, 128)) == height
+    """On 256 CUs: 128-row tiles where they take no more rounds of work items, else the tallest."""
+    assert tile_rows(pkg, rows, sum(rows), H, I, 1, fp8)[0] == height
+
+
+@pytest.mark.parametrize("H,most", [(2048, 192), (4096, 144)])
+def test_an_experts_tiles_are_equally_high(pkg, H, most):
+    """As few tiles as the height allows, in whole 16-row fragments, none a fragment per tile or more below
+    another; on streaming tiles every tile but the last is full."""
+    counts = list(range(1, 1200, 7)) + [143, 144, 145, 191, 192, 193, 288, 289, 384, 385, 576, 577, 0]
+    for part in (counts[i:i + 64] for i in range(0, len(counts), 64)):
+        got, rows = tile_rows(pkg, part, sum(part), H, 1536, 1, 1)
+        assert got in (128, most)
+        for n, h in zip(part, rows.tolist()):
+            tiles = -(-n // got)
+            assert 0 < h <= got and h % 16 == 0 and -(-n // h) == tiles
+            if tiles > 1:
+                assert h - (n - (tiles - 1) * h) < 16 * tiles
+    got, rows = tile_rows(pkg, [40] + [1] * 7, 47, H, 1536, 1, 1)
+    assert got == 16 and (rows == 16).all()
