@@ -112,12 +112,12 @@ S235B = Shape("qwen3-235b-a22b", 4096, 1536)
 # commit a71d4f3 (FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00, KiB; the factors calibrated on a 256 MiB copy);
 # commands and per-dispatch figures in profiles/grouped_gemm_hbm_traffic.md:
 #   decode 64:            FETCH 195,261 / WRITE 768 KiB
-#   prefill 4096, Zipf:   FETCH 324,585 / WRITE 25,863 KiB (build of 759266c)
+#   prefill 4096, Zipf:   FETCH 311,335 / WRITE 25,774 KiB (build of 3b05437)
 _TRAFFIC_SRC = "profiles/grouped_gemm_hbm_traffic.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, build of a71d4f3)"
-_TRAFFIC_SRC_PREFILL = _TRAFFIC_SRC.replace("a71d4f3", "759266c")
+_TRAFFIC_SRC_PREFILL = _TRAFFIC_SRC.replace("a71d4f3", "3b05437")
 MEASURED_GATE_UP_TRAFFIC = {
     ("qwen3-30b-a3b", 64): {"bytes": 195261 * 1024 * 2 + 768 * 1024, "source": _TRAFFIC_SRC},
-    ("qwen3-30b-a3b", 4096): {"bytes": 324585 * 1024 * 2 + 25863 * 1024, "source": _TRAFFIC_SRC_PREFILL},
+    ("qwen3-30b-a3b", 4096): {"bytes": 311335 * 1024 * 2 + 25774 * 1024, "source": _TRAFFIC_SRC_PREFILL},
 }
 
 

@@ -5,11 +5,12 @@
 // a tile, an expert of 129 .. 192 rows takes its weights through LDS twice).
 //
 // Bound by the stream of weights up to about 128 rows per expert (Qwen3-30B-A3B, 300 tokens: gate_up
-// 403 MB in 77.5 us, 5.2 TB/s), by the matrix cores and the LDS reads under them beyond.  Against one
-// 8-wave group with two register sets of fragments on 128-row tiles, experts layer at 301 tokens 145.5 ->
-// 136.9 us, uniform 2048 tokens 250 -> 216 us (its 129 .. 160-row experts were two tiles each),
-// Zipf-routed 4096 tokens 371.6 -> 370.8 us; bf16 experts, 1700 tokens 359 -> 343 us (with the separate
-// combine's 6 us of it).
+// 403 MB in 75.6 us, 5.3 TB/s), beyond by the issue of the operand DMA, which stretches a compute phase of
+// 785 cycles (768 of MFMAs) to 1265.  Against one 8-wave group with two register sets of fragments on
+// 128-row tiles, gate_up + down: 300 tokens 80.4 + 46.9 -> 75.6 + 44.4 us, uniform 2048 tokens 132 + 80 ->
+// 101 + 63 us (its 129 .. 160-row experts were two tiles each), Zipf-routed 4096 tokens 183 + 128 -> 170 +
+// 108 us; bf16 experts, 1700 tokens 203 + 117 -> 196 + 114 us, 300 tokens level (184 + 82: rows of 4 KB meet
+// on the same memory channels).
 //
 // The two wave groups (waves 0-3 and 4-7: one wave of each on every SIMD) run the same program half a
 // K block apart: while one issues the MFMAs of a K block (a compute phase), the other reads its next

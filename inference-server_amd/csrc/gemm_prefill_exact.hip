@@ -13,8 +13,8 @@
 // accumulators (160 registers) are what fits; what the K loop can work out anew (fresh_tid, LDS
 // addresses) is not kept in registers.
 //
-// Qwen3-235B-A22B: gate_up 706 -> 545 us and down 376 -> 277 us at 2048 tokens, 480 -> 334 us (1.6 GB of
-// weights, 4.8 TB/s) and 245 -> 156 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
+// Qwen3-235B-A22B: gate_up 687 -> 522 us and down 362 -> 272 us at 2048 tokens, 468 -> 332 us (1.6 GB of
+// weights, 4.8 TB/s) and 237 -> 157 us at 300; bound by the matrix cores (the bf16 MFMAs of 2048 tokens take
 // 165 us in gate_up at their full rate) and the waits of each quarter's LDS reads, below about 64 rows
 // per expert by the stream of weights.
 //
